@@ -1,5 +1,5 @@
-// gt_batched_f64.hip -- the FP64 (reference-exact) instantiations of the
-// HALFSPLIT strip kernels (gt_strip_impl.h), and the launch plan.
+// gt_batched_f64.hip -- the launch plan of the HALFSPLIT strip kernels
+// (gt_strip_impl.h) and the choice of their instantiation.
 #include "gt_strip_impl.h"
 
 namespace gt {
@@ -23,10 +23,13 @@ bool fused_supported(int hscheme, int vscheme) {
 template void strip_plan<double>(FusedArgs<double>&, int);
 template void strip_plan<float>(FusedArgs<float>&, int);
 
+hipError_t launch_fused_f64_g1(hipStream_t st, const FusedArgs<double>& a);
+hipError_t launch_fused_f64_g2(hipStream_t st, const FusedArgs<double>& a);
+hipError_t launch_fused_f64_adv(hipStream_t st, const FusedArgs<double>& a);
+
 hipError_t launch_fused_f64(hipStream_t st, const FusedArgs<double>& a, int group, bool adv) {
-  if (adv) return dispatch_scheme<double, 1, true, true>(st, a);
-  if (group == 2) return dispatch_scheme<double, 2, true, false>(st, a);
-  return dispatch_scheme<double, 1, true, false>(st, a);
+  if (adv) return launch_fused_f64_adv(st, a);
+  return group == 2 ? launch_fused_f64_g2(st, a) : launch_fused_f64_g1(st, a);
 }
 
 }  // namespace gt

@@ -52,8 +52,60 @@ __device__ __forceinline__ double rcp_nr(double x) {
   return __builtin_fma(r, e, r);
 }
 
+// ---- the divisions of the exact flavour ----------------------------------------
+// The compiler's a/b is v_div_scale (twice), v_rcp, two Newton steps for
+// y = 1/b, q0 = a*y, r = a - b*q0, q = q0 + r*y (v_div_fmas) and v_div_fixup:
+// 11 instructions.  Where nothing needs scaling the scale and fixup steps
+// pass their operands through, so the Newton steps and the last three
+// operations alone give the same bits, and y is formed once for every
+// quotient over the same b (the cell updates of the tracers, P2-PDM's
+// 2r/(cfl+1e-10), the division by dx).  What scaling guards against shows in
+// the remainder r, which is exact for a normal quotient of normal operands:
+// a tiny numerator (below ~2^-969) leaves it denormal; an infinity, a NaN, a
+// zero or denormal b or an overflow leaves it infinite or NaN.  DivNewton
+// collects that test over the lanes whose quotient is used, and a strip in
+// which it fired is marched again with DivFull.  (A zero numerator gives +0
+// where the full sequence keeps its sign.  |b| stays below 2^1021.)
+struct Den {
+  double b, y;
+};
+struct DivFull {
+  __device__ __forceinline__ Den den(double b) const { return {b, 0.0}; }
+  __device__ __forceinline__ double over(double a, const Den& d, bool) const { return a / d.b; }
+  __device__ __forceinline__ double div(double a, double b, bool) const { return a / b; }
+  __device__ __forceinline__ void pin() const {}
+};
+struct DivNewton {
+  uint64_t bad = 0;    // the lanes it fired on, up to the last pin()
+  bool fired = false;  // and since
+  __device__ __forceinline__ Den den(double b) const {
+    double y = __builtin_amdgcn_rcp(b);
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+    return {b, y};
+  }
+  // a/b; used: whether this lane's quotient reaches a result
+  __device__ __forceinline__ double over(double a, const Den& d, bool used) {
+    constexpr int kNanInfDenorm = 0x1 | 0x2 | 0x4 | 0x10 | 0x80 | 0x200;
+    const double q0 = a * d.y;
+    const double r = __builtin_fma(-d.b, q0, a);
+    fired |= used & __builtin_amdgcn_class(r, kNanInfDenorm);
+    return __builtin_fma(r, d.y, q0);
+  }
+  __device__ __forceinline__ double div(double a, double b, bool used) {
+    return over(a, den(b), used);
+  }
+  // ends a section of the row: the tests of the section's remainders stay in
+  // it (left to the compiler they gather at the row's end and keep every
+  // remainder in registers until there)
+  __device__ __forceinline__ void pin() {
+    bad |= __builtin_amdgcn_ballot_w64(fired);
+    asm volatile("" : "+s"(bad));
+    fired = false;
+  }
+};
+
 // ---- one face of a sweep -----------------------------------------------------
-enum : uint8_t { F_NONE = 0, F_LEFT = 1, F_LEFT_LIM = 2, F_RIGHT = 3, F_RIGHT_LIM = 4 };
 
 template <bool EXACT>
 struct FaceC;
@@ -61,7 +113,8 @@ struct FaceC;
 template <>
 struct FaceC<true> {
   double vel, cfl, Dv, E;  // E = 2/(1-cfl), P2-PDM's third bound, formed once
-  uint8_t code;
+  Den c1;                  // cfl + 1e-10, the denominator of its first
+  bool active, left, lim;  // carries a flux, goes right (upwind cell on the left), is limited
 };
 // fast: vel = 0 for an inactive face, g = 0 where the limiter does not apply
 template <>
@@ -74,65 +127,76 @@ struct FaceC<false> {
 // the fast path dti/dlen and AH/dlen (0 without diffusion)
 struct FaceK {
   double dti, dlen, cscale, kscale;
+  Den len;  // dlen as a denominator
 };
 __device__ __forceinline__ FaceK face_k(double dti, double dlen, double AH) {
-  return {dti, dlen, dti / dlen, AH > 0.0 ? AH / dlen : 0.0};
+  return {dti, dlen, dti / dlen, AH > 0.0 ? AH / dlen : 0.0, DivNewton{}.den(dlen)};
 }
 
 // face constants from the transport (vel), layer height (Dv) and masks;
 // lim_l/lim_r: the flux mask of the upwind neighbour allows the limiter
 // (adv_split_u.F90:219-265, adv_split_v.F90:77-119)
-template <int SCH>
+template <int SCH, typename Div>
 __device__ __forceinline__ void face_setup(FaceC<true>& fc, bool active, bool lim_l, bool lim_r,
-                                           double vel, double Dv, const FaceK& k) {
+                                           double vel, double Dv, const FaceK& k, Div& dv) {
   // The exact path is branch-free like the fast one: every operand is formed
   // and the result selected, so the division chains of neighbouring faces and
   // tracers share one basic block and interleave; a lane whose value is not
   // selected may compute inf or NaN, which is never used.  One division
   // chain serves both directions: the reference's vel/Dv*dti/dlen going
   // right, -vel/Dv*dti/dlen going left, with the operand selected first.
-  const double dti = k.dti, dlen = k.dlen;
   fc.vel = vel;
   fc.Dv = Dv;
   const bool left = vel > 0.0;
-  const bool lim = active && SCH != UPSTREAM && (left ? lim_l : lim_r);
-  fc.code = !active ? F_NONE : (left ? (lim ? F_LEFT_LIM : F_LEFT) : (lim ? F_RIGHT_LIM : F_RIGHT));
-  const double c = (left ? vel : -vel) / Dv * dti / dlen;
+  const bool lim = active & (SCH != UPSTREAM) & (left ? lim_l : lim_r);
+  fc.active = active;
+  fc.left = left;
+  fc.lim = lim;
+  const double c = dv.over(dv.div(left ? vel : -vel, Dv, lim) * k.dti, k.len, lim);
   fc.cfl = lim ? c : 0.0;
-  fc.E = SCH == P2_PDM ? 2.0 / (1.0 - fc.cfl) : 0.0;
+  if constexpr (SCH == P2_PDM) {
+    fc.E = dv.div(2.0, 1.0 - fc.cfl, lim);
+    fc.c1 = dv.den(fc.cfl + 1.e-10);
+  } else {
+    fc.E = 0.0;
+    fc.c1 = {1.0, 1.0};
+  }
 }
 
 // adv_interfacial_reconstruction (src/2d/advection.F90:806-845), branch-free:
 // every operation of reconstruct() in its order, P2-PDM's 2/(1-cfl) taken
 // from the face (E) instead of formed per tracer.  Returns the limited value
-// and sets take where the reference returns it (deltaf*deltafu > 0 for the
-// TVD schemes, always for P2, never for upstream) -- fu otherwise -- so the
-// caller folds this choice into its own select of the face's value
-template <int SCH>
-__device__ __forceinline__ double reconstruct_bf(double cfl, double E, double fuu, double fu,
-                                                 double fd, bool& take) {
+// and sets take where the reference returns it (lim, the limiter applies,
+// and deltaf*deltafu > 0 for the TVD schemes, lim for P2, never for upstream)
+// -- fu otherwise -- so the caller folds this choice into its own select of
+// the face's value
+template <int SCH, typename Div>
+__device__ __forceinline__ double reconstruct_bf(double cfl, double E, const Den& c1, double fuu,
+                                                 double fu, double fd, bool lim, bool& take,
+                                                 Div& dv) {
   const double deltaf = fd - fu;
   const double deltafu = fu - fuu;
   if constexpr (SCH == UPSTREAM) {
-    (void)E; (void)cfl;
+    (void)E; (void)cfl; (void)c1; (void)lim; (void)dv;
     take = false;
     return fu;
   } else if constexpr (SCH == P2) {
-    (void)E;
-    take = true;
+    (void)E; (void)c1; (void)dv;
+    take = lim;
     return reconstruct_p2<double>(cfl, fu, deltafu, deltaf);
   } else {
     // The reference's min/max are the hardware's: where the result is
     // selected (deltaf*deltafu > 0) the ratio is positive and, with
     // cfl >= 0, no operand is NaN and no two are zeros of opposite sign, so
     // v_min_f64 / v_max_f64 pick the operand the comparison form picks
-    const double ratio = deltafu / deltaf;
+    take = lim & (deltaf * deltafu > 0.0);
+    const double ratio = dv.div(deltafu, deltaf, take);
     double limiter;
     if constexpr (SCH == P2_PDM) {
       const double one6th = 1.0 / 6.0;
       const double x = one6th * (1.0 - 2.0 * cfl);
       limiter = (0.5 + x) + (0.5 - x) * ratio;
-      limiter = __builtin_fmin(__builtin_fmin(2.0 * ratio / (cfl + 1.e-10), limiter), E);
+      limiter = __builtin_fmin(__builtin_fmin(dv.over(2.0 * ratio, c1, take), limiter), E);
     } else if constexpr (SCH == SUPERBEE) {
       (void)E;
       limiter = __builtin_fmax(__builtin_fmin(2.0 * ratio, 1.0), __builtin_fmin(ratio, 2.0));
@@ -140,16 +204,15 @@ __device__ __forceinline__ double reconstruct_bf(double cfl, double E, double fu
       (void)E;
       limiter = __builtin_fmin(__builtin_fmin(2.0 * ratio, 0.5 * (1.0 + ratio)), 2.0);
     }
-    take = deltaf * deltafu > 0.0;
     return fu + 0.5 * limiter * (1.0 - cfl) * deltaf;
   }
 }
 
-template <int SCH>
+template <int SCH, typename Div>
 __device__ __forceinline__ void face_setup(FaceC<false>& fc, bool active, bool lim_l, bool lim_r,
-                                           double vel, double Dv, const FaceK& k) {
+                                           double vel, double Dv, const FaceK& k, Div&) {
   const bool right = !(vel > 0.0);
-  const bool lim = active && SCH != UPSTREAM && (right ? lim_r : lim_l);
+  const bool lim = active & (SCH != UPSTREAM) & (right ? lim_r : lim_l);
   // the Courant number feeds FP32 arithmetic only: formed in FP32
   const float c0 =
       __builtin_fabsf((float)vel) * (float)k.cscale * __builtin_amdgcn_rcpf((float)Dv);
@@ -172,9 +235,11 @@ __device__ __forceinline__ void face_setup(FaceC<false>& fc, bool active, bool l
 // On the lanes that take the limited value deltaf and deltafu share a sign,
 // and the branch terms of deltaf < 0 are those of |deltaf|, |deltafu|
 // negated, each rounding alike, so the max there is minus the min over the
-// magnitudes: one min (abs taken as operand modifiers) and the sign folded
-// into g give bit for bit the min/max selected by the sign.  No divergent
-// branch; fused multiply-adds are written out where they shorten the chain.
+// magnitudes: one min (abs taken as operand modifiers) whose sign is flipped
+// where deltaf is negative (one three-operand bit operation) gives bit for
+// bit the min/max selected by the sign.  (Not a copied sign: P2-PDM's terms
+// are negative above Courant number 1.)  No divergent branch; fused
+// multiply-adds are written out where they shorten the chain.
 template <int SCH>
 __device__ __forceinline__ float rec_fast(float fuu, float fu, float fd, float g, float A,
                                           float al, float E) {
@@ -197,8 +262,9 @@ __device__ __forceinline__ float rec_fast(float fuu, float fu, float fd, float g
       const float a2 = 2.0f * adu, b2 = 2.0f * adf, h = 0.5f * (adf + adu);
       m = __builtin_fminf(__builtin_fminf(a2, h), b2);
     }
-    const float gs = df > 0.0f ? g : -g;
-    const float r = __builtin_fmaf(gs, m, fu);
+    const uint32_t ms = __builtin_bit_cast(uint32_t, m) ^
+                        (__builtin_bit_cast(uint32_t, df) & 0x80000000u);
+    const float r = __builtin_fmaf(g, __builtin_bit_cast(float, ms), fu);
     return df * du > 0.0f ? r : fu;
   }
 }
@@ -206,26 +272,24 @@ __device__ __forceinline__ float rec_fast(float fuu, float fu, float fd, float g
 // flux through the face between cells X and X+1 of a sweep, from the cells
 // X-1, X, X+1, X+2 (fm1, f0, fp1, fp2)
 // DIFF: horizontal diffusion on (AH > 0), fixed at compile time
-template <typename TF, int SCH, bool DIFF>
+template <typename TF, int SCH, bool DIFF, typename Div>
 __device__ __forceinline__ TF face_flux(const FaceC<true>& fc, TF fm1, TF f0, TF fp1, TF fp2,
-                                        double AH, double dlen) {
+                                        double AH, const FaceK& k, Div& dv) {
   // upwind operands selected first, then one reconstruction for both
-  // directions (left: fm1, f0, fp1; right: fp2, fp1, f0), selected by the
-  // face code (branch-free, see face_setup)
-  const bool left = fc.code <= F_LEFT_LIM;
-  const TF fuu = left ? fm1 : fp2, fd = left ? fp1 : f0;
-  const TF fu0 = left ? f0 : fp1;
+  // directions (left: fm1, f0, fp1; right: fp2, fp1, f0; branch-free, see
+  // face_setup)
+  const TF fuu = fc.left ? fm1 : fp2, fd = fc.left ? fp1 : f0;
+  const TF fu0 = fc.left ? f0 : fp1;
   bool take;
-  const TF rr = reconstruct_bf<SCH>(fc.cfl, fc.E, fuu, fu0, fd, take);
-  const TF fu = ((fc.code == F_LEFT_LIM || fc.code == F_RIGHT_LIM) && take) ? rr : fu0;
-  TF fl = fc.vel * fu;
-  if constexpr (DIFF) fl = fl - AH * fc.Dv * (fp1 - f0) / dlen;
-  return fc.code == F_NONE ? TF(0) : fl;
+  const TF rr = reconstruct_bf<SCH>(fc.cfl, fc.E, fc.c1, fuu, fu0, fd, fc.lim, take, dv);
+  TF fl = fc.vel * (take ? rr : fu0);
+  if constexpr (DIFF) fl = fl - dv.over(AH * fc.Dv * (fp1 - f0), k.len, fc.active);
+  return fc.active ? fl : TF(0);
 }
 
-template <typename TF, int SCH, bool DIFF>
+template <typename TF, int SCH, bool DIFF, typename Div>
 __device__ __forceinline__ TF face_flux(const FaceC<false>& fc, TF fm1, TF f0, TF fp1, TF fp2,
-                                        double /*AH*/, double /*dlen*/) {
+                                        double /*AH*/, const FaceK&, Div&) {
   const TF fuu = fc.right ? fp2 : fm1;
   const TF fu0 = fc.right ? fp1 : f0;
   const TF fd = fc.right ? f0 : fp1;
@@ -240,12 +304,14 @@ __device__ __forceinline__ TF face_flux(const FaceC<false>& fc, TF fm1, TF f0, T
 // (adv_split_u.F90:267-286), in the reference's order (EXACT); computed on
 // every lane and selected by upd (advn_out is 0 where the cell is not
 // updated)
-__device__ __forceinline__ double cell_update_exact(bool upd, double Dio, double Dn, double fo,
+template <typename Div>
+__device__ __forceinline__ double cell_update_exact(bool upd, double Dio, const Den& Dn, double fo,
                                                     double Fc, double Fm, double dlen,
-                                                    double ard1, double dt, double* advn_out) {
+                                                    double ard1, double dt, double* advn_out,
+                                                    Div& dv) {
   const double advn = 0.5 * (Fc * dlen - Fm * dlen) * ard1;
   *advn_out = upd ? advn : 0.0;
-  const double fn = (Dio * fo - dt * advn) / Dn;
+  const double fn = dv.over(Dio * fo - dt * advn, Dn, upd);
   return upd ? fn : fo;
 }
 
@@ -254,12 +320,13 @@ __device__ __forceinline__ double cell_update_exact(bool upd, double Dio, double
 // heights (Dio-Dn taken in FP64, then rounded) and shared by the tracers
 // (CellK); the bracket is a small correction, so their few FP32 roundings
 // are far below the final rounding of fo + correction.
+// A cell that is not updated has zero factors, which leave fo as it is.
 struct CellK {
   float am1, b;
 };
-__device__ __forceinline__ CellK cell_factors(double Dio, double Dn, double dtc) {
+__device__ __forceinline__ CellK cell_factors(bool upd, double Dio, double Dn, double dtc) {
   const float r = __builtin_amdgcn_rcpf((float)Dn);
-  return {(float)(Dio - Dn) * r, (float)dtc * r};
+  return {upd ? (float)(Dio - Dn) * r : 0.0f, upd ? (float)dtc * r : 0.0f};
 }
 __device__ __forceinline__ float cell_update_fast(const CellK& k, float fo, float Fc, float Fm) {
   return fo + __builtin_fmaf(fo, k.am1, -(Fc - Fm) * k.b);
@@ -271,6 +338,7 @@ struct WFace;
 template <>
 struct WFace<true> {
   double w, cfl, E;
+  Den c1;  // as in FaceC
 };
 template <>
 struct WFace<false> {
@@ -278,16 +346,23 @@ struct WFace<false> {
 };
 
 // face k+1/2 of a column: w = ww(k), cfl from the layer heights either side
-template <int SCH>
+// (used: whether the face carries a flux that reaches a result)
+template <int SCH, typename Div>
 __device__ __forceinline__ void wface_setup(WFace<true>& wf, double w, double dt, double Dlo,
-                                            double Dhi) {
+                                            double Dhi, bool used, Div& dv) {
   wf.w = w;
-  wf.cfl = __builtin_fabs(w) * dt / (0.5 * (Dlo + Dhi));
-  wf.E = SCH == P2_PDM ? 2.0 / (1.0 - wf.cfl * 1.0) : 0.0;
+  wf.cfl = dv.div(__builtin_fabs(w) * dt, 0.5 * (Dlo + Dhi), used);
+  if constexpr (SCH == P2_PDM) {
+    wf.E = dv.div(2.0, 1.0 - wf.cfl * 1.0, used);
+    wf.c1 = dv.den(wf.cfl * 1.0 + 1.e-10);
+  } else {
+    wf.E = 0.0;
+    wf.c1 = {1.0, 1.0};
+  }
 }
-template <int SCH>
+template <int SCH, typename Div>
 __device__ __forceinline__ void wface_setup(WFace<false>& wf, double w, double dt, double Dlo,
-                                            double Dhi) {
+                                            double Dhi, bool, Div&) {
   const float c =
       __builtin_fabsf((float)w) * (float)(2.0 * dt) * __builtin_amdgcn_rcpf((float)(Dlo + Dhi));
   wf.w = (float)w;
@@ -297,34 +372,22 @@ __device__ __forceinline__ void wface_setup(WFace<false>& wf, double w, double d
   wf.E = 2.0f * __builtin_amdgcn_rcpf(1.0f - c);
 }
 
-// flux at face k+1/2 from the levels k-1..k+2 (the limiter applies above
-// level 1-kshift going up and below kmax-1 going down)
-template <typename TF, int SCH, bool EXACT>
-__device__ __forceinline__ TF wflux(const WFace<EXACT>& wf, int k, int kshift, int kmax, TF fkm1,
-                                    TF fk, TF fk1, TF fk2) {
-  TF fu, fuu = TF(0), fd = TF(0);
-  bool lim = false;
-  if (wf.w > 0) {
-    fu = fk;
-    if (SCH != UPSTREAM) lim = k > 1 - kshift;
-    if (lim) { fuu = fkm1; fd = fk1; }
-  } else {
-    fu = fk1;
-    if (SCH != UPSTREAM) lim = k < kmax - 1;
-    if (lim) { fuu = fk2; fd = fk; }
-  }
-  if constexpr (EXACT) {
-    bool take;
-    const TF rr = reconstruct_bf<SCH>(wf.cfl * 1.0, wf.E, fuu, fu, fd, take);
-    fu = (lim && take) ? rr : fu;
-  } else {
-    fu = rec_fast<SCH>(fuu, fu, fd, lim ? wf.g : 0.0f, wf.A, wf.al, wf.E);
-  }
-  return TF(wf.w) * fu;
+// flux at face k+1/2 from the levels k-1..k+2; lim_up / lim_dn: whether the
+// limiter applies going up / down at this face (above level 1-kshift, below
+// kmax-1).  Branch-free, as the horizontal faces
+template <int SCH, typename Div>
+__device__ __forceinline__ double wflux_exact(const WFace<true>& wf, bool lim_up, bool lim_dn,
+                                              double fkm1, double fk, double fk1, double fk2,
+                                              Div& dv) {
+  const bool up = wf.w > 0.0;
+  const double fu = up ? fk : fk1, fuu = up ? fkm1 : fk2, fd = up ? fk1 : fk;
+  bool take;
+  const double rr = reconstruct_bf<SCH>(wf.cfl * 1.0, wf.E, wf.c1, fuu, fu, fd,
+                                        up ? lim_up : lim_dn, take, dv);
+  return wf.w * (take ? rr : fu);
 }
 
-// fast form of wflux: every operand formed, the limiter switched off by g = 0
-// (lim_up / lim_dn: whether it applies going up / down at this face)
+// the same in FP32, the limiter switched off by g = 0
 template <int SCH>
 __device__ __forceinline__ float wflux_fast(const WFace<false>& wf, bool lim_up, bool lim_dn,
                                             float fkm1, float fk, float fk1, float fk2) {
@@ -418,34 +481,28 @@ __device__ __forceinline__ void sto(T* base, uint32_t off, T v) {
 }
 
 // The row march is unrolled four times: the four-row windows rotate by
-// renaming (logical row q of step s lives in slot (s+q)&3), and the inputs of
-// a row are loaded one step ahead into one of two row buffers (FP64) or at
-// the start of its step (FP32, below).  Loads read
+// renaming (logical row q of step s lives in slot (s+q)&3).  Loads read
 // valid addresses everywhere (cell 0 outside the array, the group's last
-// tracer past its end, level K for a level outside 0..kmax); only the flags
-// are masked, since every other value of a cell outside the array, or of a
+// tracer past its end, level K for a missing level); only the flags are
+// masked, since every other value of a cell outside the array, or of a
 // missing level, reaches discarded results only.
 
-// FP64 (the exact flavour) loads the inputs of a row one step ahead into the
-// other of two row buffers; FP32 loads them where the step starts: without
-// the second buffer's registers the FP32 kernels run one more wavefront per
-// SIMD (uv 129 -> 101, wvu 229 -> 159 VGPRs at 9 tracers), which hides more
-// (batched step 2.80 -> 2.74 ms), while FP64 loses more than it gains
-// (advection 0.46 -> 0.49 ms with 140 instead of 182 VGPRs in wvu)
+// FP64 loads a row's inputs while the row before it is computed, each tracer
+// into the registers its sub-step has just read and the shared fields once
+// the row's faces are set up, so the lookahead costs no second buffer (400 x
+// 400 x 40 x 2 tracers: 376 us against 387 with two row buffers in the u/v
+// kernel and the shared fields loaded where a row starts).  FP32 loads where
+// the row starts: its kernels issue VALU instructions in three of four cycles
+// and the longer live ranges only cost them a wavefront or spills (18 tracers
+// on eight subdomains: 2.55 ms, against 3.2 ms with the lookahead).
 template <typename TF>
-constexpr bool kRowAhead = std::is_same<TF, double>::value;
-// the w kernel's shared fields of a row (masks, w, heights, the v and u
-// transports) with its tracers, two rows ahead (true), or where the row's
-// step starts (false): with the tracers alone ahead the FP64 w kernel holds
-// 161 instead of 179 VGPRs and runs 3 wavefronts per SIMD instead of 2
-// (headline step 0.592 -> 0.587 ms); the u/v kernel keeps both ahead (103
-// instead of 113 VGPRs would leave it at 4 wavefronts per SIMD)
-template <typename TF>
-constexpr bool kWvuSharedAhead = false;
+constexpr bool kRowAhead = sizeof(TF) == 8;
 
 // ---- kernel 1: u/2 then v/2 at level L ------------------------------------------------
-template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF>
-__global__ __launch_bounds__(256) void k_strip_uv(FusedArgs<TF> A) {
+// Div: the divisions of the exact flavour; dv tells whether one left their
+// range
+template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF, typename Div>
+__device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
   StripItem it;
   if (!strip_item<0>(A, it)) return;
   const FusedDomain<TF>& a = A.doms[it.dom];
@@ -486,21 +543,24 @@ __global__ __launch_bounds__(256) void k_strip_uv(FusedArgs<TF> A) {
   // and y-3
   struct Row {
     int fl;
-    double ho, uu, hu, vv, vvm, hv;
+    double ho, uu, hu, vv, hv;
     TF f[G];
   };
-  auto load_row = [&](int y, Row& r) {
-    const uint32_t c = cell(y), c2 = cell(y - 2), c3 = cell(y - 3);
-    const uint32_t b = c * (uint32_t)sizeof(TF), b8 = c * 8u;
+  auto load_shared = [&](int y, Row& r) {
+    const uint32_t c = cell(y), c2 = cell(y - 2);
+    const uint32_t b8 = c * 8u;
     r.fl = flags[c];
     r.ho = ldo(ho, b8);
     r.uu = ldo(uu, b8);
     r.hu = ldo(hu, b8);
     r.vv = ldo(vv, c2 * 8u);
-    r.vvm = ldo(vv, c3 * 8u);
     r.hv = ldo(hv, c2 * 8u);
+  };
+  auto load_f = [&](int y, Row& r, int g) { r.f[g] = ldo(fin_g[g], cell(y) * (uint32_t)sizeof(TF)); };
+  auto load_row = [&](int y, Row& r) {
+    load_shared(y, r);
 #pragma unroll
-    for (int g = 0; g < G; g++) r.f[g] = ldo(fin_g[g], b);
+    for (int g = 0; g < G; g++) load_f(y, r, g);
   };
 
   int flw[4] = {0, 0, 0, 0};
@@ -508,6 +568,7 @@ __global__ __launch_bounds__(256) void k_strip_uv(FusedArgs<TF> A) {
   double a1w[ADV ? 4 : 1][G];
   TF f1w[G][4];
   TF fvp[G];  // v flux through the face below the row being updated
+  double vvp = 0.0;  // the v transport there
 #pragma unroll
   for (int g = 0; g < G; g++) {
     fvp[g] = TF(0);
@@ -521,8 +582,13 @@ __global__ __launch_bounds__(256) void k_strip_uv(FusedArgs<TF> A) {
       for (int g = 0; g < G; g++) a1w[q][g] = 0.0;
   }
 
-  auto step = [&](auto slot, Row& buf, int s) {
+  // one row of the march; VF / VR: whether the v face and the v row of the
+  // step exist (they start with the fourth and fifth row).  Known at compile
+  // time, and every store waits for the end of the row, so the row is one
+  // basic block in which the tracers' chains interleave
+  auto step = [&](auto slot, auto vfc, auto vrc, Row& buf, int s) {
     constexpr int R = decltype(slot)::value;
+    constexpr bool VF = decltype(vfc)::value, VR = decltype(vrc)::value;
     constexpr int w0 = R & 3, w1 = (R + 1) & 3, w2 = (R + 2) & 3, w3 = (R + 3) & 3;
     const int y = y0 - 2 + s;
     if constexpr (!kRowAhead<TF>) load_row(y, buf);
@@ -532,95 +598,119 @@ __global__ __launch_bounds__(256) void k_strip_uv(FusedArgs<TF> A) {
     // ---- u/2 on row y: shared part
     const int flm = from_lower_lane(fl), flp = from_upper_lane(fl);
     FaceC<EXACT> fu;
-    face_setup<SCH>(fu, fo & MB_UFLUX, flm & MB_UFLUX, flp & MB_UFLUX, buf.uu, buf.hu, ku);
+    face_setup<SCH>(fu, fo & MB_UFLUX, flm & MB_UFLUX, flp & MB_UFLUX, buf.uu, buf.hu, ku,
+                    dv);
     const double uum = from_lower_lane(buf.uu);
     const bool updu = fo & MB_UUPD;
     const double D0 = buf.ho;
     double D1 = D0;
     D1 = sel(updu, D0 - dth * (buf.uu * dy - uum * dy) * ard1, D0);
     CellK k1{};
-    if constexpr (!EXACT) k1 = cell_factors(D0, D1, dtcu);
+    Den e1{}, e2{};  // D1, D2 as denominators (EXACT)
+    if constexpr (EXACT) e1 = dv.den(D1);
+    else k1 = cell_factors(updu, D0, D1, dtcu);
     flw[w3] = fo;
     d1w[w3] = D1;
 
     // ---- v/2 on row yv = y-2: shared part (faces from row y0-1 on)
     const int yv = y - 2;
-    const bool vface = s >= 3, vrow = s >= 4;
     FaceC<EXACT> fv;
     bool updv = false;
     double D2 = d1w[w1];
     CellK k2{};
-    if (vface) {
-      face_setup<SCH>(fv, (flw[w1] & MB_VFLUX) && yv >= isub && yv <= NY - 2 - isub,
-                      flw[w0] & MB_VFLUX, flw[w2] & MB_VFLUX, buf.vv, buf.hv, kv);
-      updv = (flw[w1] & MB_VUPD) && yv >= 1 + isub && yv <= NY - 2 - isub;
-      D2 = sel(updv, d1w[w1] - dth * (buf.vv * dx - buf.vvm * dx) * ard1, D2);
-      if constexpr (!EXACT) k2 = cell_factors(d1w[w1], D2, dtcv);
+    if constexpr (VF) {
+      const bool yface = yv >= isub && yv <= NY - 2 - isub;
+      face_setup<SCH>(fv, yface & ((flw[w1] & MB_VFLUX) != 0), flw[w0] & MB_VFLUX,
+                      flw[w2] & MB_VFLUX, buf.vv, buf.hv, kv, dv);
+      updv = (yface && yv >= 1 + isub) & ((flw[w1] & MB_VUPD) != 0);
+      D2 = sel(updv, d1w[w1] - dth * (buf.vv * dx - vvp * dx) * ard1, D2);
+      if constexpr (EXACT) e2 = dv.den(D2);
+      else k2 = cell_factors(updv, d1w[w1], D2, dtcv);
     }
-    const bool st_ok = vrow && (flw[w1] & MB_XOUT) && yv < NY;
+    const bool st_ok = (VR && yv >= y0 && yv < NY) & ((flw[w1] & MB_XOUT) != 0);
     const uint32_t cv = (uint32_t)(x + NX * yv);
+    TF res[G];
+    double a2v = 0.0;
+    vvp = buf.vv;
+    if constexpr (kRowAhead<TF>) load_shared(y + 1, buf);
 
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-      // u/2 on row y (adv_split_u.F90:219-286)
+    // u/2 on row y (adv_split_u.F90:219-286)
+    auto sub_u = [&](int g) {
       const TF fc = buf.f[g];
       const TF fm1 = from_lower_lane(fc), fp1 = from_upper_lane(fc);
       const TF fp2 = from_upper_lane(fp1);
-      const TF Fu = face_flux<TF, SCH, DIFF>(fu, fm1, fc, fp1, fp2, AH, dx);
+      const TF Fu = face_flux<TF, SCH, DIFF>(fu, fm1, fc, fp1, fp2, AH, ku, dv);
       const TF Fum = from_lower_lane(Fu);
       double advu = 0.0;
       TF F1 = fc;
       if constexpr (EXACT) {
-        F1 = cell_update_exact(updu, D0, D1, fc, Fu, Fum, dy, ard1, dt, &advu);
+        F1 = cell_update_exact(updu, D0, e1, fc, Fu, Fum, dy, ard1, dt, &advu, dv);
       } else {
-        const TF u = cell_update_fast(k1, fc, Fu, Fum);
-        F1 = updu ? u : fc;
+        F1 = cell_update_fast(k1, fc, Fu, Fum);
       }
       f1w[g][w3] = F1;
       if constexpr (ADV) a1w[w3][g] = 0.0 + advu;
-      // v/2 on row yv (adv_split_v.F90:77-131)
-      if (vface) {
-        const TF Fv =
-            face_flux<TF, SCH, DIFF>(fv, f1w[g][w0], f1w[g][w1], f1w[g][w2], f1w[g][w3], AH, dy);
-        if (vrow) {
+      if constexpr (kRowAhead<TF>) load_f(y + 1, buf, g);
+    };
+    // v/2 on row yv (adv_split_v.F90:77-131)
+    auto sub_v = [&](int g) {
+      if constexpr (VF) {
+        const TF Fv = face_flux<TF, SCH, DIFF>(fv, f1w[g][w0], f1w[g][w1], f1w[g][w2], f1w[g][w3],
+                                               AH, kv, dv);
+        if constexpr (VR) {
           double advv = 0.0;
           TF F2 = f1w[g][w1];
           if constexpr (EXACT) {
-            F2 = cell_update_exact(updv, d1w[w1], D2, F2, Fv, fvp[g], dx, ard1, dt, &advv);
+            F2 = cell_update_exact(updv, d1w[w1], e2, F2, Fv, fvp[g], dx, ard1, dt, &advv, dv);
           } else {
-            const TF u = cell_update_fast(k2, F2, Fv, fvp[g]);
-            F2 = updv ? u : F2;
+            F2 = cell_update_fast(k2, F2, Fv, fvp[g]);
           }
-          if (st_ok && g < ntr) sto(f2_g[g], cv * (uint32_t)sizeof(TF), F2);
+          res[g] = F2;
           if constexpr (ADV) {
-            if (st_ok && g == 0) sto(a2, cv * 8u, a1w[w1][0] + advv);
+            if (g == 0) a2v = a1w[w1][0] + advv;
           }
         }
         fvp[g] = Fv;
       }
+    };
+    // FP64 a sub-step at a time, so that its tracers' division chains
+    // interleave; FP32 a tracer at a time, for fewer live registers
+    if constexpr (EXACT) {
+#pragma unroll
+      for (int g = 0; g < G; g++) sub_u(g);
+      dv.pin();
+#pragma unroll
+      for (int g = 0; g < G; g++) sub_v(g);
+      dv.pin();
+    } else {
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        sub_u(g);
+        sub_v(g);
+      }
     }
-    if (st_ok && it.grp == 0) sto(d2, cv * 8u, D2);
-    if constexpr (kRowAhead<TF>) load_row(y + 2, buf);
+    // (past the group's last tracer the pointers and values repeat it)
+    if (VR && st_ok) {
+#pragma unroll
+      for (int g = 0; g < G; g++) sto(f2_g[g], cv * (uint32_t)sizeof(TF), res[g]);
+      if constexpr (ADV) sto(a2, cv * 8u, a2v);
+      if (it.grp == 0) sto(d2, cv * 8u, D2);
+    }
   };
 
-  if constexpr (kRowAhead<TF>) {
-    Row ra, rb;
-    load_row(y0 - 2, ra);
-    load_row(y0 - 1, rb);
-    for (int s = 0; s < nsteps; s += 4) {
-      step(Slot<0>{}, ra, s);
-      step(Slot<1>{}, rb, s + 1);
-      step(Slot<2>{}, ra, s + 2);
-      step(Slot<3>{}, rb, s + 3);
-    }
-  } else {
-    Row r;
-    for (int s = 0; s < nsteps; s += 4) {
-      step(Slot<0>{}, r, s);
-      step(Slot<1>{}, r, s + 1);
-      step(Slot<2>{}, r, s + 2);
-      step(Slot<3>{}, r, s + 3);
-    }
+  constexpr std::true_type on{};
+  constexpr std::false_type off{};
+  Row r;
+  if constexpr (kRowAhead<TF>) load_row(y0 - 2, r);
+  step(Slot<0>{}, off, off, r, 0);
+  step(Slot<1>{}, off, off, r, 1);
+  step(Slot<2>{}, off, off, r, 2);
+  step(Slot<3>{}, on, off, r, 3);
+  for (int s = 4; s < nsteps; s += 4) {
+    step(Slot<0>{}, on, on, r, s);
+    step(Slot<1>{}, on, on, r, s + 1);
+    step(Slot<2>{}, on, on, r, s + 2);
+    step(Slot<3>{}, on, on, r, s + 3);
   }
 
   // level 0 of the work fields (the second kernel reads levels K-2..K+2 of
@@ -640,8 +730,8 @@ __global__ __launch_bounds__(256) void k_strip_uv(FusedArgs<TF> A) {
 // ---- kernel 2: w, then v/2 and u/2 at level K -------------------------------------------
 // BUD: some domain of the launch forms its budgets in the step (the
 // variant without them carries none of their code or registers)
-template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF, bool BUD>
-__global__ __launch_bounds__(256) void k_strip_wvu(FusedArgs<TF> A) {
+template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF, bool BUD, typename Div>
+__device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
   StripItem it;
   if (!strip_item<1>(A, it)) return;
   const FusedDomain<TF>& a = A.doms[it.dom];
@@ -682,8 +772,9 @@ __global__ __launch_bounds__(256) void k_strip_wvu(FusedArgs<TF> A) {
   uint32_t lvo[5];
 #pragma unroll
   for (int m = 0; m < 5; m++) {
+    // (level 0 takes part with kshift only; a caller may leave it unset)
     const int l = K - 2 + m;
-    lvo[m] = (uint32_t)(((l >= 0 && l <= kmax) ? l : K) * NXY * (long)sizeof(TF));
+    lvo[m] = (uint32_t)(((l >= 1 - kshift && l <= kmax) ? l : K) * NXY * (long)sizeof(TF));
   }
   const bool has_kp1 = K < kmax;
   // d2 at K-1, K, K+1 and ww at K-1, K from one base each (level K-1) and
@@ -703,14 +794,11 @@ __global__ __launch_bounds__(256) void k_strip_wvu(FusedArgs<TF> A) {
   // y-2 (v also y-3)
   struct Row {
     int fl;
-    double wwK, wwKm1, dKm1, dK, dKp1, vv, vvm, hv, uu, hu, a2;
+    double wwK, wwKm1, dKm1, dK, dKp1, vv, hv, uu, hu, a2;
     TF f[G][5];
   };
-  // the row's shared fields and its tracers, loaded apart: the tracers run
-  // ahead of the arithmetic (kRowAhead), the shared fields only as far as
-  // kWvuSharedAhead says
   auto load_shared = [&](int y, Row& r) {
-    const uint32_t c = cell(y), c2 = cell(y - 2), c3 = cell(y - 3);
+    const uint32_t c = cell(y), c2 = cell(y - 2);
     const uint32_t b8 = c * 8u, b82 = c2 * 8u;
     r.fl = flags[c];
     r.wwK = ldo(wwKm1, b8 + lstep);
@@ -719,25 +807,20 @@ __global__ __launch_bounds__(256) void k_strip_wvu(FusedArgs<TF> A) {
     r.dK = ldo(dKm1, b8 + lstep);
     r.dKp1 = ldo(dKm1, b8 + lup);
     r.vv = ldo(vv, b82);
-    r.vvm = ldo(vv, c3 * 8u);
     r.hv = ldo(hv, b82);
     r.uu = ldo(uu, b82);
     r.hu = ldo(hu, b82);
     if constexpr (ADV) r.a2 = ldo(a2, b8);
   };
-  auto load_f = [&](int y, Row& r) {
+  auto load_f = [&](int y, Row& r, int g) {
     const uint32_t b = cell(y) * (uint32_t)sizeof(TF);
-    uint32_t lb[5];
 #pragma unroll
-    for (int m = 0; m < 5; m++) lb[m] = b + lvo[m];
-#pragma unroll
-    for (int g = 0; g < G; g++)
-#pragma unroll
-      for (int m = 0; m < 5; m++) r.f[g][m] = ldo(f2_g[g], lb[m]);
+    for (int m = 0; m < 5; m++) r.f[g][m] = ldo(f2_g[g], b + lvo[m]);
   };
   auto load_row = [&](int y, Row& r) {
     load_shared(y, r);
-    load_f(y, r);
+#pragma unroll
+    for (int g = 0; g < G; g++) load_f(y, r, g);
   };
 
   int flw[4] = {0, 0, 0, 0}, fow[4] = {0, 0, 0, 0};
@@ -754,7 +837,8 @@ __global__ __launch_bounds__(256) void k_strip_wvu(FusedArgs<TF> A) {
 #pragma unroll
     for (int q = 0; q <= G; q++) bsh[wv][q][lane] = 0.0;
   }
-  TF fvp[G];
+  TF fvp[G];  // as in the first kernel
+  double vvp = 0.0;
 #pragma unroll
   for (int g = 0; g < G; g++) {
     fvp[g] = TF(0);
@@ -768,166 +852,185 @@ __global__ __launch_bounds__(256) void k_strip_wvu(FusedArgs<TF> A) {
       for (int g = 0; g < G; g++) a3w[q][g] = 0.0;
   }
 
-  auto step = [&](auto slot, Row& buf, int s) {
+  // one row of the march (VF, VR and the stores as in the first kernel)
+  auto step = [&](auto slot, auto vfc, auto vrc, Row& buf, int s) {
     constexpr int R = decltype(slot)::value;
+    constexpr bool VF = decltype(vfc)::value, VR = decltype(vrc)::value;
     constexpr int w0 = R & 3, w1 = (R + 1) & 3, w2 = (R + 2) & 3, w3 = (R + 3) & 3;
     const int y = y0 - 2 + s;
-    if constexpr (!kRowAhead<TF>) {
-      load_row(y, buf);
-    } else if constexpr (!kWvuSharedAhead<TF>) {
-      load_shared(y, buf);
-    }
+    if constexpr (!kRowAhead<TF>) load_row(y, buf);
     const int fl = (y >= 0 && y < NY) ? (buf.fl & cb.xin) : 0;  // raw masks of the cell
     const int fo = (fl | MB_XOUT) & cb.xm;                      // ... with the column bounds
 
     // ---- w on row y: shared part
-    const bool wcol = (fo & MB_WCOL) && y <= NY - 2;
-    const bool wupd = wcol && kdo;
+    const bool wcol = (y <= NY - 2) & ((fo & MB_WCOL) != 0);
+    const bool wupd = wcol & kdo;
     const double D2K = buf.dK;
     double D3 = D2K;
     D3 = sel(wupd, D2K - dt * (buf.wwK - buf.wwKm1), D2K);
     CellK k3{};
-    if constexpr (!EXACT) k3 = cell_factors(D2K, D3, dt);
+    Den e3{}, e4{}, e5{};  // D3, D4, D5 as denominators (EXACT)
+    if constexpr (EXACT) e3 = dv.den(D3);
+    else k3 = cell_factors(wupd, D2K, D3, dt);
     WFace<EXACT> wfk, wfp;
-    wface_setup<SCH>(wfk, buf.wwK, dt, D2K, buf.dKp1);
-    wface_setup<SCH>(wfp, buf.wwKm1, dt, buf.dKm1, D2K);
+    const bool onk = wcol & wk_on, onp = wcol & wp_on;
+    wface_setup<SCH>(wfk, onk ? buf.wwK : 0.0, dt, D2K, buf.dKp1, onk, dv);
+    wface_setup<SCH>(wfp, onp ? buf.wwKm1 : 0.0, dt, buf.dKm1, D2K, onp, dv);
     flw[w3] = fl;
     fow[w3] = fo;
     d3w[w3] = D3;
 
     // ---- v/2 and u/2 on row yv = y-2: shared part
     const int yv = y - 2;
-    const bool vface = s >= 3, vrow = s >= 4;
     FaceC<EXACT> fv, fu;
     bool updv = false, updu = false;
     double D4 = d3w[w1], D5 = d3w[w1];
     CellK k4{}, k5{};
-    if (vface) {
-      face_setup<SCH>(fv, (flw[w1] & MB_VFLUX) && yv >= isub && yv <= NY - 2 - isub,
-                      flw[w0] & MB_VFLUX, flw[w2] & MB_VFLUX, buf.vv, buf.hv, kv);
-      updv = (flw[w1] & MB_VUPD) && yv >= 1 + isub && yv <= NY - 2 - isub;
-      D4 = sel(updv, d3w[w1] - dth * (buf.vv * dx - buf.vvm * dx) * ard1, D4);
-      if constexpr (!EXACT) k4 = cell_factors(d3w[w1], D4, dtcv);
+    if constexpr (VF) {
+      const bool yface = yv >= isub && yv <= NY - 2 - isub;
+      face_setup<SCH>(fv, yface & ((flw[w1] & MB_VFLUX) != 0), flw[w0] & MB_VFLUX,
+                      flw[w2] & MB_VFLUX, buf.vv, buf.hv, kv, dv);
+      updv = (yface && yv >= 1 + isub) & ((flw[w1] & MB_VUPD) != 0);
+      D4 = sel(updv, d3w[w1] - dth * (buf.vv * dx - vvp * dx) * ard1, D4);
+      if constexpr (EXACT) e4 = dv.den(D4);
+      else k4 = cell_factors(updv, d3w[w1], D4, dtcv);
     }
-    if (vrow) {
+    if constexpr (VR) {
       const int flv = flw[w1], fov = fow[w1];
       const int flm = from_lower_lane(flv), flp = from_upper_lane(flv);
-      face_setup<SCH>(fu, fov & MB_UFLUX, flm & MB_UFLUX, flp & MB_UFLUX, buf.uu, buf.hu, ku);
+      face_setup<SCH>(fu, fov & MB_UFLUX, flm & MB_UFLUX, flp & MB_UFLUX, buf.uu, buf.hu, ku,
+                    dv);
       const double uum = from_lower_lane(buf.uu);
       updu = fov & MB_UUPD;
-      D5 = D4;
       D5 = sel(updu, D4 - dth * (buf.uu * dy - uum * dy) * ard1, D4);
-      if constexpr (!EXACT) k5 = cell_factors(D4, D5, dtcu);
+      if constexpr (EXACT) e5 = dv.den(D5);
+      else k5 = cell_factors(updu, D4, D5, dtcu);
     }
-    const bool st_ok = vrow && (fow[w1] & MB_XOUT) && yv < NY;
+    const bool st_ok = (VR && yv >= y0 && yv < NY) & ((fow[w1] & MB_XOUT) != 0);
     const uint32_t cv = (uint32_t)(x + NX * yv);
-    // interior water cell of the mass and volume budgets
-    const bool bcell = bud && st_ok && (flw[w1] & MB_WCOL) && x >= 2 && x <= NX - 3 &&
-                       yv >= 2 && yv <= NY - 3;
+    TF res[G], f4[G];
+    double a5v = 0.0, a4[ADV ? G : 1];
+    [[maybe_unused]] const double A2 = ADV ? buf.a2 : 0.0;
+    vvp = buf.vv;
+    if constexpr (kRowAhead<TF>) load_shared(y + 1, buf);
 
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-      // w on row y (adv_split_w.F90:249-300); the level below 1 is zero in
-      // the argument, level kmax+1 is never read by the limiter
+    // w on row y (adv_split_w.F90:249-300); a face that does not exist has
+    // w = 0, and what its operands read in place of a missing level reaches
+    // no limiter
+    auto sub_w = [&](int g) {
       const TF fKm2 = buf.f[g][0], fKm1 = buf.f[g][1], fK = buf.f[g][2];
       const TF fKp1 = buf.f[g][3], fKp2 = buf.f[g][4];
-      TF wprev = TF(0), wk = TF(0);
-      if constexpr (EXACT) {
-        const TF p =
-            wflux<TF, SCH, EXACT>(wfp, K - 1, kshift, kmax, K > 1 ? fKm2 : TF(0), fKm1, fK, fKp1);
-        const TF q = wflux<TF, SCH, EXACT>(wfk, K, kshift, kmax, fKm1, fK, fKp1, fKp2);
-        wprev = (wcol && wp_on) ? p : TF(0);
-        wk = (wcol && wk_on) ? q : TF(0);
-      } else {
-        const TF p = wflux_fast<SCH>(wfp, limp_up, limp_dn, K > 1 ? fKm2 : TF(0), fKm1, fK, fKp1);
-        const TF q = wflux_fast<SCH>(wfk, limk_up, limk_dn, fKm1, fK, fKp1, fKp2);
-        wprev = (wcol && wp_on) ? p : TF(0);
-        wk = (wcol && wk_on) ? q : TF(0);
-      }
       TF F3 = fK;
       double advw = 0.0;
       if constexpr (EXACT) {
+        const TF wprev =
+            wflux_exact<SCH>(wfp, limp_up & onp, limp_dn & onp, fKm2, fKm1, fK, fKp1, dv);
+        const TF wk =
+            wflux_exact<SCH>(wfk, limk_up & onk, limk_dn & onk, fKm1, fK, fKp1, fKp2, dv);
         const double aw = 1.0 * (wk - wprev);
-        const double f3 = (D2K * fK - dt * aw) / D3;
+        const double f3 = dv.over(D2K * fK - dt * aw, e3, wupd);
         advw = wupd ? aw : 0.0;
         F3 = wupd ? f3 : fK;
       } else {
-        const TF u = cell_update_fast(k3, fK, wk, wprev);
-        F3 = wupd ? u : fK;
+        const TF wprev = wflux_fast<SCH>(wfp, limp_up, limp_dn, fKm2, fKm1, fK, fKp1);
+        const TF wk = wflux_fast<SCH>(wfk, limk_up, limk_dn, fKm1, fK, fKp1, fKp2);
+        F3 = cell_update_fast(k3, fK, wk, wprev);
       }
       f3w[g][w3] = F3;
-      if constexpr (ADV) a3w[w3][g] = buf.a2 + advw;
-      if (vface) {
-        // v/2 on row yv (adv_split_v.F90:77-131)
-        const TF Fv =
-            face_flux<TF, SCH, DIFF>(fv, f3w[g][w0], f3w[g][w1], f3w[g][w2], f3w[g][w3], AH, dy);
-        if (vrow) {
-          double advv = 0.0, advu = 0.0;
+      if constexpr (ADV) a3w[w3][g] = A2 + advw;
+      if constexpr (kRowAhead<TF>) load_f(y + 1, buf, g);
+    };
+    // v/2 on row yv (adv_split_v.F90:77-131)
+    auto sub_v = [&](int g) {
+      if constexpr (VF) {
+        const TF Fv = face_flux<TF, SCH, DIFF>(fv, f3w[g][w0], f3w[g][w1], f3w[g][w2], f3w[g][w3],
+                                               AH, kv, dv);
+        if constexpr (VR) {
+          double advv = 0.0;
           TF F4 = f3w[g][w1];
           if constexpr (EXACT) {
-            F4 = cell_update_exact(updv, d3w[w1], D4, F4, Fv, fvp[g], dx, ard1, dt, &advv);
+            F4 = cell_update_exact(updv, d3w[w1], e4, F4, Fv, fvp[g], dx, ard1, dt, &advv, dv);
           } else {
-            const TF u = cell_update_fast(k4, F4, Fv, fvp[g]);
-            F4 = updv ? u : F4;
+            F4 = cell_update_fast(k4, F4, Fv, fvp[g]);
           }
-          // u/2 on row yv (adv_split_u.F90:219-286)
-          const TF fm1 = from_lower_lane(F4), fp1 = from_upper_lane(F4);
-          const TF fp2 = from_upper_lane(fp1);
-          const TF Fu = face_flux<TF, SCH, DIFF>(fu, fm1, F4, fp1, fp2, AH, dx);
-          const TF Fum = from_lower_lane(Fu);
-          TF F5 = F4;
-          if constexpr (EXACT) {
-            F5 = cell_update_exact(updu, D4, D5, F4, Fu, Fum, dy, ard1, dt, &advu);
-          } else {
-            const TF u = cell_update_fast(k5, F4, Fu, Fum);
-            F5 = updu ? u : F4;
-          }
-          if (st_ok && g < ntr) sto(fo_g[g], cv * (uint32_t)sizeof(TF), F5);
-          if (bcell) bsh[wv][g][lane] = __builtin_fma(D5, (double)F5, bsh[wv][g][lane]);
-          if constexpr (ADV) {
-            if (st_ok && g == 0 && a.advres) {
-              const double A4 = a3w[w1][0] + advv;
-              a.advres[oK + cv] = A4 + advu;
-            }
-          }
+          f4[g] = F4;
+          if constexpr (ADV) a4[g] = a3w[w1][g] + advv;
         }
         fvp[g] = Fv;
       }
+    };
+    // u/2 on row yv (adv_split_u.F90:219-286)
+    auto sub_u = [&](int g) {
+      if constexpr (VR) {
+        const TF F4 = f4[g];
+        double advu = 0.0;
+        const TF fm1 = from_lower_lane(F4), fp1 = from_upper_lane(F4);
+        const TF fp2 = from_upper_lane(fp1);
+        const TF Fu = face_flux<TF, SCH, DIFF>(fu, fm1, F4, fp1, fp2, AH, ku, dv);
+        const TF Fum = from_lower_lane(Fu);
+        TF F5 = F4;
+        if constexpr (EXACT) {
+          F5 = cell_update_exact(updu, D4, e5, F4, Fu, Fum, dy, ard1, dt, &advu, dv);
+        } else {
+          F5 = cell_update_fast(k5, F4, Fu, Fum);
+        }
+        res[g] = F5;
+        if constexpr (ADV) {
+          if (g == 0) a5v = a4[0] + advu;
+        }
+      }
+    };
+    // (the order as in the first kernel)
+    if constexpr (EXACT) {
+#pragma unroll
+      for (int g = 0; g < G; g++) sub_w(g);
+      dv.pin();
+#pragma unroll
+      for (int g = 0; g < G; g++) sub_v(g);
+      dv.pin();
+#pragma unroll
+      for (int g = 0; g < G; g++) sub_u(g);
+      dv.pin();
+    } else {
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        sub_w(g);
+        sub_v(g);
+        sub_u(g);
+      }
     }
-    if (st_ok && it.grp == 0 && hires) sto(hires, cv * 8u, D5);
-    if (bcell && it.grp == 0) bsh[wv][G][lane] += D5;
-    if constexpr (kRowAhead<TF>) {
-      if constexpr (kWvuSharedAhead<TF>) {
-        load_row(y + 2, buf);
-      } else {
-        load_f(y + 2, buf);
+    // (past the group's last tracer the pointers and values repeat it)
+    if (VR && st_ok) {
+#pragma unroll
+      for (int g = 0; g < G; g++) sto(fo_g[g], cv * (uint32_t)sizeof(TF), res[g]);
+      if constexpr (ADV) {
+        if (a.advres) a.advres[oK + cv] = a5v;
+      }
+      if (it.grp == 0 && hires) sto(hires, cv * 8u, D5);
+      // interior water cell of the mass and volume budgets
+      if (BUD && bud && (flw[w1] & MB_WCOL) && x >= 2 && x <= NX - 3 && yv >= 2 &&
+          yv <= NY - 3) {
+#pragma unroll
+        for (int g = 0; g < G; g++)
+          bsh[wv][g][lane] = __builtin_fma(D5, (double)res[g], bsh[wv][g][lane]);
+        if (it.grp == 0) bsh[wv][G][lane] += D5;
       }
     }
   };
 
-  if constexpr (kRowAhead<TF>) {
-    Row ra, rb;
-    if constexpr (kWvuSharedAhead<TF>) {
-      load_row(y0 - 2, ra);
-      load_row(y0 - 1, rb);
-    } else {
-      load_f(y0 - 2, ra);
-      load_f(y0 - 1, rb);
-    }
-    for (int s = 0; s < nsteps; s += 4) {
-      step(Slot<0>{}, ra, s);
-      step(Slot<1>{}, rb, s + 1);
-      step(Slot<2>{}, ra, s + 2);
-      step(Slot<3>{}, rb, s + 3);
-    }
-  } else {
-    Row r;
-    for (int s = 0; s < nsteps; s += 4) {
-      step(Slot<0>{}, r, s);
-      step(Slot<1>{}, r, s + 1);
-      step(Slot<2>{}, r, s + 2);
-      step(Slot<3>{}, r, s + 3);
-    }
+  constexpr std::true_type on{};
+  constexpr std::false_type off{};
+  Row r;
+  if constexpr (kRowAhead<TF>) load_row(y0 - 2, r);
+  step(Slot<0>{}, off, off, r, 0);
+  step(Slot<1>{}, off, off, r, 1);
+  step(Slot<2>{}, off, off, r, 2);
+  step(Slot<3>{}, on, off, r, 3);
+  for (int s = 4; s < nsteps; s += 4) {
+    step(Slot<0>{}, on, on, r, s);
+    step(Slot<1>{}, on, on, r, s + 1);
+    step(Slot<2>{}, on, on, r, s + 2);
+    step(Slot<3>{}, on, on, r, s + 3);
   }
 
   // the budget partials of this strip-level: the lanes' sums added over the
@@ -966,6 +1069,58 @@ __global__ __launch_bounds__(256) void k_strip_wvu(FusedArgs<TF> A) {
         if (a.advres) a.advres[c] = 0.0;
       }
     }
+  }
+}
+
+// ---- the kernels --------------------------------------------------------------------
+// The exact flavour marches a strip with the short divisions and, where one of
+// them left its range, again with the full ones: a call, so that the rarely
+// taken march shares no registers with the other (inlined it took the FP64
+// kernels from 126 and 189 to 250 VGPRs).  The call takes the kernel
+// argument's address and makes it uniform again.
+// Wavefronts per SIMD the kernels must leave room for: u/v FP64 4, the others
+// 3.  Left to itself the compiler trades them for instruction-level
+// parallelism, and 400 x 400 x 40 x 2 FP64 tracers take 419 us (3 and 2)
+// against 400; more than these spill in the row loop (FP32 at 4: 2.6 -> 3.2
+// ms on the 18-tracer batch).
+template <typename TF>
+constexpr int kWavesUv = sizeof(TF) == 8 ? 4 : 3;
+constexpr int kWavesWvu = 3;
+template <typename TF>
+__device__ __forceinline__ const FusedArgs<TF>& uniform_args(uint64_t p) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)p);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(p >> 32));
+  using Arg = const __attribute__((address_space(4))) FusedArgs<TF>;
+  return *(const FusedArgs<TF>*)(Arg*)(((uint64_t)hi << 32) | lo);
+}
+template <typename TF, int SCH, int G, bool ADV, bool DIFF>
+__device__ __attribute__((noinline)) void strip_uv_full(uint64_t args) {
+  DivFull dv;
+  strip_uv<TF, SCH, G, true, ADV, DIFF>(uniform_args<TF>(args), dv);
+}
+template <typename TF, int SCH, int G, bool ADV, bool DIFF, bool BUD>
+__device__ __attribute__((noinline)) void strip_wvu_full(uint64_t args) {
+  DivFull dv;
+  strip_wvu<TF, SCH, G, true, ADV, DIFF, BUD>(uniform_args<TF>(args), dv);
+}
+
+template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF>
+__global__ __launch_bounds__(256, kWavesUv<TF>) void k_strip_uv(FusedArgs<TF> A) {
+  std::conditional_t<EXACT, DivNewton, DivFull> dv;
+  strip_uv<TF, SCH, G, EXACT, ADV, DIFF>(A, dv);
+  if constexpr (EXACT) {
+    if (dv.bad)
+      strip_uv_full<TF, SCH, G, ADV, DIFF>((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
+  }
+}
+
+template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF, bool BUD>
+__global__ __launch_bounds__(256, kWavesWvu) void k_strip_wvu(FusedArgs<TF> A) {
+  std::conditional_t<EXACT, DivNewton, DivFull> dv;
+  strip_wvu<TF, SCH, G, EXACT, ADV, DIFF, BUD>(A, dv);
+  if constexpr (EXACT) {
+    if (dv.bad)
+      strip_wvu_full<TF, SCH, G, ADV, DIFF, BUD>((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
   }
 }
 

@@ -102,16 +102,15 @@ __device__ __forceinline__ FaceC<EXACT> face_at(const Sweep& s, int X, long x2, 
   const bool lim_l = SCH != UPSTREAM && X >= 1 && (flags[x2 - s.st] & s.mflux);
   const bool lim_r = SCH != UPSTREAM && (flags[x2 + s.st] & s.mflux);
   FaceC<EXACT> fc;
-  face_setup<SCH>(fc, active, lim_l, lim_r, vel[o + x2], Dv[o + x2], k);
+  DivFull dv;
+  face_setup<SCH>(fc, active, lim_l, lim_r, vel[o + x2], Dv[o + x2], k, dv);
   return fc;
 }
 
 // a face that carries no flux (outside the sweep's face range)
 template <bool EXACT>
 __device__ __forceinline__ FaceC<EXACT> no_face() {
-  FaceC<EXACT> fc{};
-  if constexpr (EXACT) fc.code = F_NONE;
-  return fc;
+  return FaceC<EXACT>{};
 }
 
 // the loads of row Y of a v march: face Y's transport, layer height and
@@ -146,7 +145,8 @@ __device__ __forceinline__ FaceC<EXACT> vface(const Dims& d, int Y, const VRaw& 
   const bool lim_l = SCH != UPSTREAM && Y >= 1 && (r.fm & MB_VFLUX);
   const bool lim_r = SCH != UPSTREAM && (r.fp & MB_VFLUX);
   FaceC<EXACT> fc;
-  face_setup<SCH>(fc, active, lim_l, lim_r, r.vel, r.Dv, k);
+  DivFull dv;
+  face_setup<SCH>(fc, active, lim_l, lim_r, r.vel, r.Dv, k, dv);
   return fc;
 }
 
@@ -160,7 +160,7 @@ struct CellOp<false> {
   float am1 = 0.0f, b = 0.0f;
   // dtc = dt*splitfac*dlen*ard1 (dt for w)
   __device__ static CellOp make(double Dio, double Dn, double dtc) {
-    const CellK k = cell_factors(Dio, Dn, dtc);
+    const CellK k = cell_factors(true, Dio, Dn, dtc);
     CellOp c;
     c.am1 = k.am1;
     c.b = k.b;
@@ -188,7 +188,8 @@ struct CellOp<true> {
   __device__ double h_step(double fo, double Fc, double Fm, double dt, double dlen,
                            double ard1) const {
     double advn;
-    return cell_update_exact(true, Dio, Dn, fo, Fc, Fm, dlen, ard1, dt, &advn);
+    DivFull dv;
+    return cell_update_exact(true, Dio, dv.den(Dn), fo, Fc, Fm, dlen, ard1, dt, &advn, dv);
   }
   // adv_split_w.F90:287-294
   __device__ double w_step(double fo, double wk, double wprev, double dt) const {
@@ -298,9 +299,8 @@ __device__ __forceinline__ void face_flux_grad(const FaceC<kExact<TF>>& fc, TF f
                                                TF fp2, double AH, double dlen, TF out[4]) {
   if constexpr (kExact<TF>) {
     out[0] = out[1] = out[2] = out[3] = 0.0;
-    if (fc.code == F_NONE) return;
-    const bool left = fc.code <= F_LEFT_LIM;
-    const bool lim = fc.code == F_LEFT_LIM || fc.code == F_RIGHT_LIM;
+    if (!fc.active) return;
+    const bool left = fc.left, lim = fc.lim;
     const double fuu = left ? fm1 : fp2, fu0 = left ? f0 : fp1, fd = left ? fp1 : f0;
     const RecG<double> r =
         lim ? rec_grad_exact<SCH>(fc.cfl, fc.E, fuu, fu0, fd) : RecG<double>{0.0, 1.0, 0.0};
@@ -333,13 +333,12 @@ __device__ __forceinline__ void face_flux_grad(const FaceC<kExact<TF>>& fc, TF f
 // the w flux at face K (K+1/2) from the levels K-1..K+2, and its partials;
 // lim_up / lim_dn: whether the limiter applies going up / down
 template <typename TF, int SCH>
-__device__ __forceinline__ TF w_flux(const WFace<kExact<TF>>& wf, int K, int kshift, int kmax,
-                                     bool lim_up, bool lim_dn, TF fkm1, TF fk, TF fk1, TF fk2) {
+__device__ __forceinline__ TF w_flux(const WFace<kExact<TF>>& wf, bool lim_up, bool lim_dn,
+                                     TF fkm1, TF fk, TF fk1, TF fk2) {
   if constexpr (kExact<TF>) {
-    (void)lim_up; (void)lim_dn;
-    return wflux<TF, SCH, true>(wf, K, kshift, kmax, fkm1, fk, fk1, fk2);
+    DivFull dv;
+    return wflux_exact<SCH>(wf, lim_up, lim_dn, fkm1, fk, fk1, fk2, dv);
   } else {
-    (void)K; (void)kshift; (void)kmax;
     return wflux_fast<SCH>(wf, lim_up, lim_dn, fkm1, fk, fk1, fk2);
   }
 }
@@ -394,9 +393,11 @@ __global__ __launch_bounds__(256) void k_sub_u(Dims d, int ntr, long ts,
       for (int t = 0; t < ntr; t++) fout[t * ts + c] = fin[t * ts + c];
     return;
   }
+  const FaceK fk = face_k(0.5 * dt, dx, AH);
+  DivFull dv;
   FaceC<EX> fc = no_face<EX>();
   if (xin && x <= d.NX - 2)
-    fc = face_at<SCH, EX>(sweep(d, 0), x, c2, o, flags, uu, hu, face_k(0.5 * dt, dx, AH));
+    fc = face_at<SCH, EX>(sweep(d, 0), x, c2, o, flags, uu, hu, fk);
   const bool upd = xin && x >= 1 + isub && x <= d.NX - 2 - isub && (flags[c2] & MB_UUPD);
   CellOp<EX> cu;
   if (upd) cu = CellOp<EX>::make(Dio[c], Dn[c], dt * (0.5 * dy * ard1));
@@ -404,7 +405,7 @@ __global__ __launch_bounds__(256) void k_sub_u(Dims d, int ntr, long ts,
     const TF fx = fin[t * ts + c];
     const TF fm1 = from_lower_lane(fx), fp1 = from_upper_lane(fx);
     const TF fp2 = from_upper_lane(fp1);
-    const TF Fc = face_flux<TF, SCH, DIFF>(fc, fm1, fx, fp1, fp2, AH, dx);
+    const TF Fc = face_flux<TF, SCH, DIFF>(fc, fm1, fx, fp1, fp2, AH, fk, dv);
     const TF Fm = from_lower_lane(Fc);
     const TF u = cu.h_step(fx, Fc, Fm, dt, dy, ard1);
     if (out) fout[t * ts + c] = upd ? u : fx;
@@ -446,6 +447,7 @@ __global__ __launch_bounds__(64) void k_sub_v(Dims d, int ntr, long ts, const TF
     return;
   }
   const FaceK fk = face_k(0.5 * dt, dy, AH);
+  DivFull dv;
   const double dtc = dt * (0.5 * dx * ard1);
   auto row = [&](int y) -> long { return o + x + (long)NX * (y >= 0 && y < NY ? y : 0); };
   TF w[G][4], Fp[G];
@@ -468,7 +470,7 @@ __global__ __launch_bounds__(64) void k_sub_v(Dims d, int ntr, long ts, const TF
     if (upd) cu = CellOp<EX>::make(r.Dio, r.Dn, dtc);
 #pragma unroll
     for (int g = 0; g < G; g++) {
-      const TF F = face_flux<TF, SCH, DIFF>(fc, w[g][0], w[g][1], w[g][2], w[g][3], AH, dy);
+      const TF F = face_flux<TF, SCH, DIFF>(fc, w[g][0], w[g][1], w[g][2], w[g][3], AH, fk, dv);
       if (st && t0 + g < ntr) {
         const TF u = cu.h_step(w[g][1], F, Fp[g], dt, dx, ard1);
         fout[tb[g] + cY] = upd ? u : w[g][1];
@@ -550,16 +552,17 @@ __global__ __launch_bounds__(256) void k_sub_w(Dims d, int ntr, long ts, const T
   // so each face is evaluated once and carried up (pc).  The operands agree
   // except the one past kmax that the strip kernels substitute, which is the
   // upwind-upwind level of a downward face with the limiter off: not read.
+  DivFull dv;
   TF pc[G];
   {
     const int F = K0 - 1;  // the face below level K0
     WFace<EX> wf0;
-    wface_setup<SCH>(wf0, ww[c2 + NXY * F], dt, D2[c2 + NXY * F], d2r[0]);
+    wface_setup<SCH>(wf0, ww[c2 + NXY * F], dt, D2[c2 + NXY * F], d2r[0], true, dv);
     const bool lim_up = SCH != UPSTREAM && F > 1 - kshift;
     const bool lim_dn = SCH != UPSTREAM && F < kmax - 1;
 #pragma unroll
     for (int g = 0; g < G; g++)
-      pc[g] = w_flux<TF, SCH>(wf0, F, kshift, kmax, lim_up, lim_dn, fKm2[g], n[g][1], n[g][2],
+      pc[g] = w_flux<TF, SCH>(wf0, lim_up, lim_dn, fKm2[g], n[g][1], n[g][2],
                               K0 + 1 <= kmax ? n[g][3] : n[g][2]);
   }
   for (int K = K0; K <= K1; K++) {
@@ -569,7 +572,7 @@ __global__ __launch_bounds__(256) void k_sub_w(Dims d, int ntr, long ts, const T
     const bool limk_dn = SCH != UPSTREAM && K < kmax - 1;
     const double dk = d2r[0], dp = d2r[1];  // D2 at K, K+1
     WFace<EX> wfk;
-    wface_setup<SCH>(wfk, wr[0], dt, dk, K + 1 <= kmax ? dp : dk);
+    wface_setup<SCH>(wfk, wr[0], dt, dk, K + 1 <= kmax ? dp : dk, true, dv);
     const CellOp<EX> cw = CellOp<EX>::make(dk, d3r[0], dt);
     const bool nxt = K + 3 <= kmax;
     const long cn = c2 + NXY * (nxt ? K + 3 : kmax);
@@ -579,7 +582,7 @@ __global__ __launch_bounds__(256) void k_sub_w(Dims d, int ntr, long ts, const T
       // level K
       const TF fKm1 = n[g][1], fK = n[g][2];
       const TF fKp1 = K + 1 <= kmax ? n[g][3] : fK, fKp2 = K + 2 <= kmax ? n[g][4] : fK;
-      const TF q = w_flux<TF, SCH>(wfk, K, kshift, kmax, limk_up, limk_dn, fKm1, fK, fKp1, fKp2);
+      const TF q = w_flux<TF, SCH>(wfk, limk_up, limk_dn, fKm1, fK, fKp1, fKp2);
       const TF wprev = wp_on ? pc[g] : TF(0), wk = wk_on ? q : TF(0);
       const TF r = kdo ? cw.w_step(fK, wk, wprev, dt) : fK;
       if (t0 + g < ntr) fout[tb[g] + cK] = r;
@@ -871,7 +874,8 @@ __global__ __launch_bounds__(256) void k_sub_w_adj(Dims d, int ntr, long ts,
     // kshift and 0 without
     const bool used = Kf >= 1 || kshift;
     WFace<EX> wf;
-    wface_setup<SCH>(wf, wq[0], dt, dq[0], dq[1]);
+    DivFull dv;
+    wface_setup<SCH>(wf, wq[0], dt, dq[0], dq[1], true, dv);
     const bool lim_up = SCH != UPSTREAM && Kf > 1 - kshift;
     const bool lim_dn = SCH != UPSTREAM && Kf < kmax - 1;
 #pragma unroll

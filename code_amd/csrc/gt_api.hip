@@ -72,8 +72,8 @@ struct gt_ctx {
   int do_mirror_2d = 1;
   int fused = 1;        // use the HALFSPLIT strip kernels where they apply
   int adj_keep = -1;    // reverse mode keeps each segment's sub-step states (-1: if they fit)
-  int tile = 0;         // rows per strip of the two strip kernels (gt::strip_rows)
-  int group = 3;        // tracers per wavefront of the FP32 batched kernels
+  int tile = -1;        // rows per strip of the two strip kernels (gt::strip_rows; -1: by size)
+  int group = 0;        // tracers per wavefront of the batched kernels (0: by number and size)
   void* ws = nullptr;   // work fields of the strip kernels (grown on demand)
   size_t ws_bytes = 0;
   // coordinates(): namelist values (domain module) and the SAVE'd state
@@ -171,13 +171,6 @@ extern "C" int gt_create(gt_ctx** out, int imin, int imax, int jmin, int jmax, i
   c->d.kmax = kmax;
   c->d.NXY = (long)c->d.NX * c->d.NY;
   c->N3 = c->d.NXY * (kmax + 1);
-  // default strip height: 16 rows, or 8 where 16-row strips would give the
-  // strip kernels fewer than 4096 wavefronts (one tracer group), so a small
-  // grid still fills the chip (gt_set_tuning / gt_autotune_batch override)
-  {
-    const long items16 = (long)((c->d.NX + 59) / 60) * ((c->d.NY + 15) / 16) * (kmax + 1);
-    c->tile = items16 < 4096 ? 2 : 0;
-  }
   c->dx = dx; c->dy = dy;
   c->ard1 = 1.0 / (dx * dy);  // domain.F90:596
   const long NX = c->d.NX, NY = c->d.NY, NXY = c->d.NXY;
@@ -478,10 +471,10 @@ static size_t strip_ws_bytes(const gt_ctx* c, size_t tf_bytes, int ntracers, boo
   return sizeof(double) * (size_t)c->N3 * (adv ? 2 : 1) + tf_bytes * (size_t)c->N3 * ntracers;
 }
 
-// strip-levels of the second strip kernel at its smallest strip height (8
-// rows): the most budget partials a tuning can ask for
+// strip-levels of the second strip kernel at its smallest strip height (4
+// rows): the most budget partials a launch can ask for
 static long budget_strip_levels(const gt_ctx* c) {
-  return (long)((c->d.NX + gt::kStripOut - 1) / gt::kStripOut) * ((c->d.NY + 7) / 8) * c->kmax;
+  return (long)((c->d.NX + gt::kStripOut - 1) / gt::kStripOut) * ((c->d.NY + 3) / 4) * c->kmax;
 }
 static size_t budget_ws_bytes(const gt_ctx* c, int ntracers) {
   return sizeof(double) * 2 * (size_t)(ntracers + 1) * (size_t)budget_strip_levels(c);
@@ -767,7 +760,8 @@ extern "C" int gt_do_advection_3d(gt_ctx* c, double dt, double* f, const double*
         fill_domain<double>(c, g, &A.doms[0], f, f, 0, 1, uu, vv, ww, hu, hv, ho, hires, advres);
         A.ndom = 1;
         A.ntracers = 1;
-        gt::strip_rows(c->tile, A.rows);
+        if (c->tile >= 0) gt::strip_rows(c->tile, A.rows);
+        else gt::strip_auto_rows(A, 1);
         A.dt = dt; A.AH = AH;
         A.hscheme = hscheme; A.vscheme = vscheme; A.kshift = tag == GT_W_TAG ? 1 : 0;
         gt::strip_plan(A, 1);
@@ -1420,9 +1414,6 @@ static int batch_impl(int ndom, const gt_batch_domain* doms, int ntracers, doubl
                              AH, tag == GT_W_TAG ? 1 : 0, st));
     return GT_OK;
   }
-  // FP64: two tracers per wavefront (T and S) when there are two or more,
-  // unless the tuning asks for one
-  const int group = sizeof(TF) == 4 ? c0->group : (ntracers >= 2 && c0->group != 1 ? 2 : 1);
   for (int i = 0; i < ndom; i++) {
     gt_ctx* c = doms[i].ctx;
     TRY(ensure_ws(c, strip_ws_bytes(c, sizeof(TF), ntracers, false) +
@@ -1443,7 +1434,14 @@ static int batch_impl(int ndom, const gt_batch_domain* doms, int ntracers, doubl
     }
     A.ndom = nd;
     A.ntracers = ntracers;
-    gt::strip_rows(c0->tile, A.rows);
+    // FP64: two tracers per wavefront (T and S) when there are two or more,
+    // unless the tuning asks for one
+    // (2 is no FP32 group: 3 stands for it)
+    const int group = sizeof(TF) == 4 && c0->group ? (c0->group == 2 ? 3 : c0->group)
+                      : c0->group == 1             ? 1
+                                                   : gt::strip_auto_group(A);
+    if (c0->tile >= 0) gt::strip_rows(c0->tile, A.rows);
+    else gt::strip_auto_rows(A, group);
     A.dt = dt; A.AH = AH;
     A.hscheme = hscheme; A.vscheme = vscheme; A.kshift = tag == GT_W_TAG ? 1 : 0;
     gt::strip_plan(A, group);

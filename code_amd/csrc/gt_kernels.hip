@@ -998,18 +998,16 @@ __global__ __launch_bounds__(256) void k_budget_batch_partial(
   }
 }
 
-// one block: the npairs (hi, lo) pairs at pq in k_budget_final's order and
-// rounding; *outq = sum * area
-__device__ __forceinline__ void budget_pairs_block(long npairs, const double* __restrict__ pq,
-                                                   double area, double* outq) {
-  __shared__ double sm[2][256];
+// one block of N threads: the sum of its threads' double-doubles as a tree;
+// *outq = sum * area
+template <int N>
+__device__ __forceinline__ void budget_tree(double sh, double sl, double area, double* outq) {
+  __shared__ double sm[2][N];
   const int t = threadIdx.x;
-  double sh = 0, sl = 0;
-  for (long b = t; b < npairs; b += blockDim.x) dd_add_dd(sh, sl, pq[2 * b], pq[2 * b + 1]);
   sm[0][t] = sh;
   sm[1][t] = sl;
   __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
+  for (int s = N / 2; s > 0; s >>= 1) {
     if (t < s) {
       double a = sm[0][t], b = sm[1][t];
       dd_add_dd(a, b, sm[0][t + s], sm[1][t + s]);
@@ -1025,6 +1023,15 @@ __device__ __forceinline__ void budget_pairs_block(long npairs, const double* __
   *outq = p + pe;
 }
 
+// one block: the npairs (hi, lo) pairs at pq in k_budget_final's order and
+// rounding; *outq = sum * area
+__device__ __forceinline__ void budget_pairs_block(long npairs, const double* __restrict__ pq,
+                                                   double area, double* outq) {
+  double sh = 0, sl = 0;
+  for (long b = threadIdx.x; b < npairs; b += 256) dd_add_dd(sh, sl, pq[2 * b], pq[2 * b + 1]);
+  budget_tree<256>(sh, sl, area, outq);
+}
+
 // one block per output q: out[q] from the partials of all blocks
 __global__ __launch_bounds__(256) void k_budget_batch_final(int nblocks,
                                                             const double* __restrict__ partial,
@@ -1034,8 +1041,12 @@ __global__ __launch_bounds__(256) void k_budget_batch_final(int nblocks,
 }
 
 // the budgets of several domains in one launch: nout blocks per domain, one
-// per output
-__global__ __launch_bounds__(256) void k_budget_pairs_final(BudgetPairsSet S) {
+// per output.  A block adds its pairs as double-doubles, which is a chain of
+// ~40 dependent additions per pair behind a load: 1024 threads with four sums
+// each keep 16 times the chains of one 256-thread sum in flight (1.6e5 pairs
+// per output, 2000 x 1500 x 50: 304 -> 30 us)
+constexpr int kPairThreads = 1024, kPairSums = 4;
+__global__ __launch_bounds__(kPairThreads) void k_budget_pairs_final(BudgetPairsSet S) {
   int i = 0;
   long b0 = 0;
   while (i + 1 < S.n && blockIdx.x >= b0 + S.d[i].nout) {
@@ -1044,7 +1055,21 @@ __global__ __launch_bounds__(256) void k_budget_pairs_final(BudgetPairsSet S) {
   }
   const BudgetPairs& D = S.d[i];
   const long q = blockIdx.x - b0;
-  budget_pairs_block(D.npairs, D.partial + 2 * q * D.npairs, D.area, D.out + q);
+  const double2* pq = (const double2*)(D.partial + 2 * q * D.npairs);
+  double sh[kPairSums] = {}, sl[kPairSums] = {};
+  for (long b = threadIdx.x; b < D.npairs; b += kPairThreads * kPairSums) {
+    double2 p[kPairSums];
+#pragma unroll
+    for (int m = 0; m < kPairSums; m++) {
+      const long c = b + m * kPairThreads;
+      p[m] = c < D.npairs ? pq[c] : double2{0.0, 0.0};
+    }
+#pragma unroll
+    for (int m = 0; m < kPairSums; m++) dd_add_dd(sh[m], sl[m], p[m].x, p[m].y);
+  }
+#pragma unroll
+  for (int m = 1; m < kPairSums; m++) dd_add_dd(sh[0], sl[0], sh[m], sl[m]);
+  budget_tree<kPairThreads>(sh[0], sl[0], D.area, D.out + q);
 }
 
 }  // namespace gt
@@ -1234,7 +1259,8 @@ hipError_t launch_budget_pairs_final(hipStream_t st, const BudgetPairsSet& S) {
   long nblocks = 0;
   for (int i = 0; i < S.n; i++) nblocks += S.d[i].nout;
   if (nblocks == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_budget_pairs_final, dim3((unsigned)nblocks), dim3(256), 0, st, S);
+  hipLaunchKernelGGL(k_budget_pairs_final, dim3((unsigned)nblocks), dim3(kPairThreads), 0, st,
+                     S);
   return hipGetLastError();
 }
 

@@ -480,6 +480,54 @@ static size_t budget_ws_bytes(const gt_ctx* c, int ntracers) {
   return sizeof(double) * 2 * (size_t)(ntracers + 1) * (size_t)budget_strip_levels(c);
 }
 
+// the HALFSPLIT and FULLSPLIT sub-steps of ns slices from level k0 in two
+// launches: u and v in one strip march into the work fields, then the closing
+// u half (HALFSPLIT) or the way back to the caller's arrays.  Replaces the
+// copies of Do, the cleared advective term and a launch per sub-step; needs
+// one scheme of the split family and 32-bit field offsets.
+static bool strips_2d_fit(const gt_ctx* c, int split, int scheme) {
+  return c->fused && (split == GT_FULLSPLIT || split == GT_HALFSPLIT) && split_scheme(scheme) &&
+         strip_fits(c);
+}
+static int strips_2d(gt_ctx* c, const GridMasks* g, int k0, int ns, double dt, double* f,
+                     const double* U, const double* V, const double* DU, const double* DV,
+                     const double* Do, int split, int scheme, double AH, double* Dires,
+                     double* advres) {
+  const bool half = split == GT_HALFSPLIT;
+  const long NXY = c->d.NXY, o = NXY * k0;
+  TRY(ensure_ws(c, strip_ws_bytes(c, sizeof(double), 1, advres != nullptr)));
+  gt::FusedArgs<double> A{};
+  gt::FusedDomain<double>& D = A.doms[0];
+  // the kernel's levels are 1..ns: the bases lie one slice below
+  const long b = o - NXY;
+  fill_domain<double>(c, g, &D, f + b, nullptr, 0, 1, U + b, V + b, nullptr, DU + b, DV + b,
+                      Do + b, nullptr, advres);
+  double *f2 = D.f2, *d2 = D.d2, *a2 = D.a2;
+  D.f2 = f2 - NXY;
+  D.d2 = d2 - NXY;
+  if (a2) D.a2 = a2 - NXY;
+  D.d.kmax = ns;
+  A.ndom = 1;
+  A.ntracers = 1;
+  if (c->tile >= 0) gt::strip_rows(c->tile, A.rows);
+  else gt::strip_auto_rows(A, 1);
+  A.dt = dt; A.AH = AH;
+  A.hscheme = A.vscheme = scheme;
+  A.fracu = half ? 0.5 : 1.0;
+  A.fracv = 1.0;
+  A.lev0 = 0;
+  gt::strip_plan(A, 1);
+  LCHK(gt::launch_strip_uv_f64(c->st, A, advres != nullptr));
+  double* di = Dires ? Dires + o : nullptr;
+  double* ad = advres ? advres + o : nullptr;
+  if (half)
+    LCHK(gt::launch_half_u(c->st, c->d, ns, f2, d2, a2, f + o, di, ad, U + o, DU + o, g->flags, dt,
+                           c->dx, c->dy, c->ard1, scheme, AH));
+  else
+    LCHK(gt::launch_copy3(c->st, NXY * ns, f + o, f2, di, d2, ad, a2));
+  return GT_OK;
+}
+
 // ---- advection entry points --------------------------------------------------
 __global__ void k_reconstruct_batch(int scheme, long n, const double* cfl, const double* fuu,
                                     const double* fu, const double* fd, double* out) {
@@ -643,6 +691,8 @@ extern "C" int gt_do_advection(gt_ctx* c, double dt, double* f, const double* U,
   const GridMasks* g = grid_for(c, tag);
   if (!g) return set_err(GT_EINVAL_TAG, "do_advection: tag is invalid");
   TRY(check_2d(split, scheme));
+  if (strips_2d_fit(c, split, scheme))
+    return strips_2d(c, g, 0, 1, dt, f, U, V, DU, DV, Do, split, scheme, AH, Dires, advres);
   const long n = c->d.NXY;
   ENSURE(c->slice3, 3 * n);
   double* fi = c->slice3;
@@ -698,6 +748,32 @@ extern "C" int gt_do_advection_3d(gt_ctx* c, double dt, double* f, const double*
   }
   const long N3 = c->N3, NXY = c->d.NXY;
   const int kmax = c->kmax;
+  const int itv = c->adv_ver_iterations;
+  if (hadv && !vadv && strips_2d_fit(c, split, hscheme)) {
+    if (hires) TRY(copy_d2d(c, hires, ho, NXY));
+    if (advres) HIPCHK(hipMemsetAsync(advres, 0, sizeof(double) * NXY, c->st));
+    return strips_2d(c, g, 1, kmax, dt, f, uu, vv, hu, hv, ho, split, hscheme, AH, hires, advres);
+  }
+  // FULLSPLIT: u and v in one strip march, then w (the schemes may differ)
+  if (hadv && vadv && split == GT_FULLSPLIT && strips_2d_fit(c, split, hscheme) && itv <= 1 &&
+      kmax > 1) {
+    TRY(ensure_ws(c, strip_ws_bytes(c, sizeof(double), 1, advres != nullptr)));
+    gt::FusedArgs<double> A{};
+    gt::FusedDomain<double>& D = A.doms[0];
+    fill_domain<double>(c, g, &D, f, f, 0, 1, uu, vv, ww, hu, hv, ho, hires, advres);
+    A.ndom = 1;
+    A.ntracers = 1;
+    if (c->tile >= 0) gt::strip_rows(c->tile, A.rows);
+    else gt::strip_auto_rows(A, 1);
+    A.dt = dt; A.AH = AH;
+    A.hscheme = A.vscheme = hscheme;
+    A.fracu = A.fracv = 1.0;
+    gt::strip_plan(A, 1);
+    LCHK(gt::launch_strip_uv_f64(c->st, A, advres != nullptr));
+    LCHK(gt::launch_full_w(c->st, c->d, D.f2, D.d2, D.a2, ww, ho, g->flags, f, hires, advres, dt,
+                           vscheme, tag == GT_W_TAG ? 1 : 0));
+    return GT_OK;
+  }
   double* phi = hires;
   double* padv = advres;
   if (!phi) { ENSURE(c->hi, N3); phi = c->hi; }
@@ -710,7 +786,6 @@ extern "C" int gt_do_advection_3d(gt_ctx* c, double dt, double* f, const double*
   double* tmp = c->tmp;
   // level 0 is never advanced horizontally; keep it equal in both buffers
   TRY(copy_d2d(c, tmp, f, NXY));
-  const int itv = c->adv_ver_iterations;
 
   if (!hadv) {
     if (kmax > 1) {

@@ -55,6 +55,10 @@ struct FusedArgs {
   int rows[2];     // rows per strip of the first (u/2 v/2) and second (w v/2 u/2) kernel
   double dt, AH;
   int hscheme, vscheme, kshift;
+  // FP64, first kernel: the parts of dt its u and v sub-steps advance (the
+  // second kernel's are halves), and whether it also passes level 0 on
+  double fracu = 0.5, fracv = 0.5;
+  int lev0 = 1;
 };
 
 // rows per strip for a tuning index: 0 -> 16, 1 -> 32, 2 -> 8 for both
@@ -77,5 +81,24 @@ template <typename TF>
 void strip_plan(FusedArgs<TF>& a, int group);
 hipError_t launch_fused_f64(hipStream_t st, const FusedArgs<double>& a, int group, bool adv);
 hipError_t launch_fused_f32(hipStream_t st, const FusedArgs<float>& a, int group);
+// the u and v sub-steps alone, FP64, one tracer: f2, d2 (and a2 with adv)
+// after them (u by fracu*dt, then v by fracv*dt)
+hipError_t launch_strip_uv_f64(hipStream_t st, const FusedArgs<double>& a, bool adv);
+// a u sub-step by dt/2 over the ns slices of d (f2, d2, a2 -> f, di, adv; a2
+// and adv may be NULL)
+hipError_t launch_half_u(hipStream_t st, Dims d, int ns, const double* f2, const double* d2,
+                         const double* a2, double* f, double* di, double* adv, const double* U,
+                         const double* DU, const uint8_t* flags, double dt, double dx, double dy,
+                         double ard1, int scheme, double AH);
+// n values each: f = f2, di = d2, adv = a2 (a NULL destination is left out)
+hipError_t launch_copy3(hipStream_t st, long n, double* f, const double* f2, double* di,
+                        const double* d2, double* adv, const double* a2);
+// the w sub-step by dt of FULLSPLIT (adv_ver_iterations = 1): f2, d2, a2 ->
+// f (level 0 left alone), hires and advres (all levels; each may be NULL,
+// advres with a2)
+hipError_t launch_full_w(hipStream_t st, Dims d, const double* f2, const double* d2,
+                         const double* a2, const double* ww, const double* ho,
+                         const uint8_t* flags, double* f, double* hires, double* advres,
+                         double dt, int scheme, int kshift);
 
 }  // namespace gt

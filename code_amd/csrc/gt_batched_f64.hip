@@ -80,6 +80,12 @@ template void strip_auto_rows<float>(FusedArgs<float>&, int);
 hipError_t launch_fused_f64_g1(hipStream_t st, const FusedArgs<double>& a);
 hipError_t launch_fused_f64_g2(hipStream_t st, const FusedArgs<double>& a);
 hipError_t launch_fused_f64_adv(hipStream_t st, const FusedArgs<double>& a);
+hipError_t launch_strip_uv_g1(hipStream_t st, const FusedArgs<double>& a);
+hipError_t launch_strip_uv_adv(hipStream_t st, const FusedArgs<double>& a);
+
+hipError_t launch_strip_uv_f64(hipStream_t st, const FusedArgs<double>& a, bool adv) {
+  return adv ? launch_strip_uv_adv(st, a) : launch_strip_uv_g1(st, a);
+}
 
 hipError_t launch_fused_f64(hipStream_t st, const FusedArgs<double>& a, int group, bool adv) {
   if (adv) return launch_fused_f64_adv(st, a);

@@ -300,16 +300,16 @@ __device__ __forceinline__ TF face_flux(const FaceC<false>& fc, TF fm1, TF f0, T
 }
 
 // the tracer update of one cell of a horizontal sub-step: the reference's
-// (Dio*fo - dt*advn)/Dn, advn = splitfac*(Fc*dlen - Fm*dlen)*ard1
+// (Dio*fo - dt*advn)/Dn, advn = frac*(Fc*dlen - Fm*dlen)*ard1 (frac: splitfac)
 // (adv_split_u.F90:267-286), in the reference's order (EXACT); computed on
 // every lane and selected by upd (advn_out is 0 where the cell is not
 // updated)
 template <typename Div>
 __device__ __forceinline__ double cell_update_exact(bool upd, double Dio, const Den& Dn, double fo,
-                                                    double Fc, double Fm, double dlen,
-                                                    double ard1, double dt, double* advn_out,
-                                                    Div& dv) {
-  const double advn = 0.5 * (Fc * dlen - Fm * dlen) * ard1;
+                                                    double Fc, double Fm, double frac,
+                                                    double dlen, double ard1, double dt,
+                                                    double* advn_out, Div& dv) {
+  const double advn = frac * (Fc * dlen - Fm * dlen) * ard1;
   *advn_out = upd ? advn : 0.0;
   const double fn = dv.over(Dio * fo - dt * advn, Dn, upd);
   return upd ? fn : fo;
@@ -516,9 +516,11 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
   constexpr int isub = SCH == UPSTREAM ? 0 : 1;
   const ColumnBits cb = column_bits(x, lane, NX, isub);
   const bool xout = (cb.xm & MB_XOUT) != 0;
-  const double dt = A.dt, dth = 0.5 * A.dt, dx = a.dx, dy = a.dy, ard1 = a.ard1, AH = A.AH;
+  const double dt = A.dt, dx = a.dx, dy = a.dy, ard1 = a.ard1, AH = A.AH;
+  const double fracu = EXACT ? A.fracu : 0.5, fracv = EXACT ? A.fracv : 0.5;
+  const double dtu = fracu * dt, dtv = fracv * dt;
   const double dtcu = dt * (0.5 * dy * ard1), dtcv = dt * (0.5 * dx * ard1);
-  const FaceK ku = face_k(dth, dx, AH), kv = face_k(dth, dy, AH);
+  const FaceK ku = face_k(dtu, dx, AH), kv = face_k(dtv, dy, AH);
   const long oL = NXY * (long)it.lev;
   const long ts = a.tstride;
   const TF* fin_g[G];
@@ -604,7 +606,7 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
     const bool updu = fo & MB_UUPD;
     const double D0 = buf.ho;
     double D1 = D0;
-    D1 = sel(updu, D0 - dth * (buf.uu * dy - uum * dy) * ard1, D0);
+    D1 = sel(updu, D0 - dtu * (buf.uu * dy - uum * dy) * ard1, D0);
     CellK k1{};
     Den e1{}, e2{};  // D1, D2 as denominators (EXACT)
     if constexpr (EXACT) e1 = dv.den(D1);
@@ -623,7 +625,7 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
       face_setup<SCH>(fv, yface & ((flw[w1] & MB_VFLUX) != 0), flw[w0] & MB_VFLUX,
                       flw[w2] & MB_VFLUX, buf.vv, buf.hv, kv, dv);
       updv = (yface && yv >= 1 + isub) & ((flw[w1] & MB_VUPD) != 0);
-      D2 = sel(updv, d1w[w1] - dth * (buf.vv * dx - vvp * dx) * ard1, D2);
+      D2 = sel(updv, d1w[w1] - dtv * (buf.vv * dx - vvp * dx) * ard1, D2);
       if constexpr (EXACT) e2 = dv.den(D2);
       else k2 = cell_factors(updv, d1w[w1], D2, dtcv);
     }
@@ -644,7 +646,7 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
       double advu = 0.0;
       TF F1 = fc;
       if constexpr (EXACT) {
-        F1 = cell_update_exact(updu, D0, e1, fc, Fu, Fum, dy, ard1, dt, &advu, dv);
+        F1 = cell_update_exact(updu, D0, e1, fc, Fu, Fum, fracu, dy, ard1, dt, &advu, dv);
       } else {
         F1 = cell_update_fast(k1, fc, Fu, Fum);
       }
@@ -661,7 +663,8 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
           double advv = 0.0;
           TF F2 = f1w[g][w1];
           if constexpr (EXACT) {
-            F2 = cell_update_exact(updv, d1w[w1], e2, F2, Fv, fvp[g], dx, ard1, dt, &advv, dv);
+            F2 = cell_update_exact(updv, d1w[w1], e2, F2, Fv, fvp[g], fracv, dx, ard1, dt, &advv,
+                                   dv);
           } else {
             F2 = cell_update_fast(k2, F2, Fv, fvp[g]);
           }
@@ -715,7 +718,7 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
 
   // level 0 of the work fields (the second kernel reads levels K-2..K+2 of
   // f2 and K-1..K+1 of d2 from one base): the input tracers and ho
-  if (it.lev == 1 && xout) {
+  if (A.lev0 && it.lev == 1 && xout) {
     for (int yv = y0; yv < y0 + A.rows[0] && yv < NY; yv++) {
       const uint32_t c = (uint32_t)(x + NX * yv);
       for (int g = 0; g < ntr; g++) {
@@ -949,7 +952,7 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
           double advv = 0.0;
           TF F4 = f3w[g][w1];
           if constexpr (EXACT) {
-            F4 = cell_update_exact(updv, d3w[w1], e4, F4, Fv, fvp[g], dx, ard1, dt, &advv, dv);
+            F4 = cell_update_exact(updv, d3w[w1], e4, F4, Fv, fvp[g], 0.5, dx, ard1, dt, &advv, dv);
           } else {
             F4 = cell_update_fast(k4, F4, Fv, fvp[g]);
           }
@@ -970,7 +973,7 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
         const TF Fum = from_lower_lane(Fu);
         TF F5 = F4;
         if constexpr (EXACT) {
-          F5 = cell_update_exact(updu, D4, e5, F4, Fu, Fum, dy, ard1, dt, &advu, dv);
+          F5 = cell_update_exact(updu, D4, e5, F4, Fu, Fum, 0.5, dy, ard1, dt, &advu, dv);
         } else {
           F5 = cell_update_fast(k5, F4, Fu, Fum);
         }
@@ -1138,6 +1141,27 @@ void strip_plan(FusedArgs<TF>& a, int group) {
     }
     a.nitems[p] = items;
   }
+}
+
+// the first kernel alone (its fractions in A; FP64): hscheme only
+template <typename TF, int G, bool ADV>
+hipError_t launch_uv(hipStream_t st, const FusedArgs<TF>& A) {
+  const unsigned grid = (unsigned)((((A.nitems[0] + 3) / 4 + 7) / 8) * 8);
+#define GT_UV(S)                                                                              \
+  if (A.AH > 0.0)                                                                             \
+    hipLaunchKernelGGL((k_strip_uv<TF, S, G, true, ADV, true>), dim3(grid), dim3(256), 0, st, A); \
+  else                                                                                        \
+    hipLaunchKernelGGL((k_strip_uv<TF, S, G, true, ADV, false>), dim3(grid), dim3(256), 0, st, A)
+  switch (A.hscheme) {
+    case P2_PDM: GT_UV(P2_PDM); break;
+    case SUPERBEE: GT_UV(SUPERBEE); break;
+    case MUSCL: GT_UV(MUSCL); break;
+    case P2: GT_UV(P2); break;
+    case UPSTREAM: GT_UV(UPSTREAM); break;
+    default: return hipErrorInvalidValue;
+  }
+#undef GT_UV
+  return hipGetLastError();
 }
 
 template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF>

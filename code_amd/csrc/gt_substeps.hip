@@ -189,7 +189,7 @@ struct CellOp<true> {
                            double ard1) const {
     double advn;
     DivFull dv;
-    return cell_update_exact(true, Dio, dv.den(Dn), fo, Fc, Fm, dlen, ard1, dt, &advn, dv);
+    return cell_update_exact(true, Dio, dv.den(Dn), fo, Fc, Fm, 0.5, dlen, ard1, dt, &advn, dv);
   }
   // adv_split_w.F90:287-294
   __device__ double w_step(double fo, double wk, double wprev, double dt) const {

@@ -1063,6 +1063,29 @@ extern "C" int gt_uv_advect_3d(gt_ctx* c, double dt, const double* uu, const dou
     if (!p) return set_err(GT_EARG, "gt_uv_advect_3d: NULL argument");
   if (hscheme == GT_J7) return set_err(GT_ENOTIMPL, "uv_advect_3d: J7 is not in this build");
   if (hscheme == GT_NOADV && vscheme == GT_NOADV) return GT_OK;
+  if (split == GT_HALFSPLIT && c->fused && c->adv_ver_iterations <= 1 && c->kmax > 1 &&
+      gt::fused_supported(hscheme, vscheme) && strip_fits(c)) {
+    const size_t ws = strip_ws_bytes(c, sizeof(double), 1, true);
+    TRY(ensure_ws(c, ws + sizeof(double) * (size_t)c->d.NX * (c->kmax + 1)));
+    for (int part = 0; part < 2; part++) {
+      gt::FusedArgs<double> A{};
+      fill_domain<double>(c, part == 0 ? &c->U : &c->V, &A.doms[0], nullptr, nullptr, 0, 1, uu,
+                          vv, ww, hun, hvn, ho, nullptr, part == 0 ? uuEx : vvEx);
+      A.doms[0].hn = hn;
+      A.doms[0].mrow = (double*)((char*)c->ws + ws);
+      A.ndom = 1;
+      A.ntracers = 1;
+      if (c->tile >= 0) gt::strip_rows(c->tile, A.rows);
+      else gt::strip_auto_rows(A, 1);
+      A.dt = dt;
+      A.AH = 0.0;
+      A.hscheme = hscheme; A.vscheme = vscheme;
+      A.lev0 = 0;
+      gt::strip_plan(A, 1);
+      LCHK(gt::launch_momentum_f64(c->st, A, part));
+    }
+    return GT_OK;
+  }
   ENSURE(c->mwork, 6 * c->N3);
   double* w[6];
   for (int q = 0; q < 6; q++) w[q] = c->mwork + q * c->N3;
@@ -1350,7 +1373,8 @@ extern "C" int gt_reserve(gt_ctx* c, int ntracers_f32, int ntracers_f64) {
   if (!c || ntracers_f32 < 0 || ntracers_f64 < 0)
     return set_err(GT_EARG, "gt_reserve: bad argument");
   // the batched step's work fields with room for the budgets formed in it
-  size_t ws = strip_ws_bytes(c, sizeof(double), 1, true);
+  size_t ws = strip_ws_bytes(c, sizeof(double), 1, true) +
+              sizeof(double) * (size_t)c->d.NX * (c->kmax + 1);  // (and uv_advect_3d's row)
   const size_t w32 = strip_ws_bytes(c, sizeof(float), ntracers_f32, false) +
                      (ntracers_f32 > 0 ? budget_ws_bytes(c, ntracers_f32) : 0);
   const size_t w64 = strip_ws_bytes(c, sizeof(double), ntracers_f64, false) +

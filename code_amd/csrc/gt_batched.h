@@ -32,6 +32,8 @@ struct FusedDomain {
   double* d2;         // work: layer heights after u/2 + v/2 (one field)
   double* a2;         // work (ADV): advective term accumulated over u/2 + v/2
   const double *uu, *vv, *ww, *hu, *hv, *ho;
+  const double* hn;      // momentum variants only
+  double* mrow;          // work (momentum): the U part's result on the last row, NX per level
   const uint8_t* flags;  // MB_* bits of the mask set of the grid
   double* hires;      // optional: end of the layer-height trajectory
   double* advres;     // optional (FP64, one tracer): accumulated advective term
@@ -84,6 +86,10 @@ hipError_t launch_fused_f32(hipStream_t st, const FusedArgs<float>& a, int group
 // the u and v sub-steps alone, FP64, one tracer: f2, d2 (and a2 with adv)
 // after them (u by fracu*dt, then v by fracv*dt)
 hipError_t launch_strip_uv_f64(hipStream_t st, const FusedArgs<double>& a, bool adv);
+// the HALFSPLIT step of the velocity on the U (part 0) or V (1) control
+// volumes (uv_advect_3d.F90): advres from uu, vv, ww, ho, hn, hun (as hu) and
+// hvn (as hv); hscheme == vscheme
+hipError_t launch_momentum_f64(hipStream_t st, const FusedArgs<double>& a, int part);
 // a u sub-step by dt/2 over the ns slices of d (f2, d2, a2 -> f, di, adv; a2
 // and adv may be NULL)
 hipError_t launch_half_u(hipStream_t st, Dims d, int ns, const double* f2, const double* d2,

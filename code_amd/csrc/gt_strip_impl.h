@@ -460,8 +460,11 @@ struct ColumnBits {
 __device__ __forceinline__ ColumnBits column_bits(int x, int lane, int NX, int isub) {
   const bool in = x >= 0 && x < NX;
   int xm = MB_VFLUX | MB_VUPD;
-  if (x >= isub && x <= NX - 2 - isub) xm |= MB_UFLUX;
-  if (x >= 1 + isub && x <= NX - 2 - isub) xm |= MB_UUPD;
+  // (the u faces and updates of the outermost lanes reach no written column,
+  // and what they would read beyond the wavefront is zero)
+  const bool inner = lane >= 1 && lane <= 62;
+  if (inner && x >= isub && x <= NX - 2 - isub) xm |= MB_UFLUX;
+  if (inner && x >= 1 + isub && x <= NX - 2 - isub) xm |= MB_UUPD;
   if (x <= NX - 2) xm |= MB_WCOL;
   if (lane >= 2 && lane < 2 + kStripOut) xm |= MB_XOUT;
   return {in ? x : 0, in ? 0xff : 0, in ? xm : 0};
@@ -498,10 +501,24 @@ __device__ __forceinline__ void sto(T* base, uint32_t off, T v) {
 template <typename TF>
 constexpr bool kRowAhead = sizeof(TF) == 8;
 
+// The momentum variants (MOM; FP64, one tracer): the tracer is the velocity
+// of the U (MOM = 1) or V (2) control volumes and the transports, w and layer
+// heights are averaged onto those volumes (uv_advect_3d.F90:70-92, 238-256)
+// where a row is read, instead of in a kernel of their own that writes six
+// work fields and has them read back (400 x 400 x 40, both parts: 606 us, 920
+// with the averaging kernels).
+// The caller's arrays come as uu, vv, ww, ho, hn, hu = hun and hv = hvn.  The
+// averages go to the next column (a lane move; the last column is zero) or
+// the next row (loaded; the last row of the V part starts from the U part's
+// result there, as the routine's work array does: mrow).  Only advres is
+// wanted: the second kernel leaves out the result and its last division but
+// on that row.
+enum { MOM_NONE = 0, MOM_U = 1, MOM_V = 2 };
+
 // ---- kernel 1: u/2 then v/2 at level L ------------------------------------------------
 // Div: the divisions of the exact flavour; dv tells whether one left their
 // range
-template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF, typename Div>
+template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF, int MOM, typename Div>
 __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
   StripItem it;
   if (!strip_item<0>(A, it)) return;
@@ -541,24 +558,59 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
     return (y >= 0 && y < NY) ? (uint32_t)(cb.xc + NX * y) : (uint32_t)cb.xc;
   };
 
-  // inputs of the step of row y: the u/2 row y and the v faces of rows y-2
-  // and y-3
+  // inputs of the step of row y: the u/2 row y and the v face of row y-2 (the
+  // momentum variants: the fields they are averaged from)
   struct Row {
     int fl;
     double ho, uu, hu, vv, hv;
+    double hn, uun, hun, vvc, vvn;  // MOM
     TF f[G];
   };
+  [[maybe_unused]] const double* hn = MOM ? a.hn + oL : nullptr;
   auto load_shared = [&](int y, Row& r) {
     const uint32_t c = cell(y), c2 = cell(y - 2);
-    const uint32_t b8 = c * 8u;
+    const uint32_t b8 = c * 8u, b82 = c2 * 8u;
     r.fl = flags[c];
-    r.ho = ldo(ho, b8);
     r.uu = ldo(uu, b8);
     r.hu = ldo(hu, b8);
-    r.vv = ldo(vv, c2 * 8u);
-    r.hv = ldo(hv, c2 * 8u);
+    r.vv = ldo(vv, b82);
+    if constexpr (MOM == MOM_V) {
+      const uint32_t n = cell(y + 1) * 8u, n2 = cell(y - 1) * 8u;
+      r.hv = ldo(hv, b8);
+      r.uun = ldo(uu, n);
+      r.hun = ldo(hu, n);
+      const bool last = y == NY - 1;
+      r.vvc = ldo(last ? a.mrow + (long)NX * it.lev : vv, last ? (uint32_t)cb.xc * 8u : b8);
+      r.vvn = ldo(vv, n2);
+      r.ho = ldo(ho, n2);
+      r.hn = ldo(hn, n2);
+    } else {
+      r.ho = ldo(ho, b8);
+      r.hv = ldo(hv, b82);
+      if constexpr (MOM == MOM_U) r.hn = ldo(hn, b8);
+    }
   };
-  auto load_f = [&](int y, Row& r, int g) { r.f[g] = ldo(fin_g[g], cell(y) * (uint32_t)sizeof(TF)); };
+  auto load_f = [&](int y, Row& r, int g) {
+    if constexpr (!MOM) r.f[g] = ldo(fin_g[g], cell(y) * (uint32_t)sizeof(TF));
+  };
+  // the row's transports and heights, and (momentum) its velocity
+  struct Fields {
+    double ho, uu, hu, vv, hv;
+  };
+  auto fields = [&](int y, Row& r) -> Fields {
+    if constexpr (MOM == MOM_U) {
+      r.f[0] = x <= NX - 2 ? r.uu / r.hu : 0.0;
+      return {r.hu, 0.5 * (r.uu + from_upper_lane(r.uu)), from_upper_lane(0.5 * (r.ho + r.hn)),
+              0.5 * (r.vv + from_upper_lane(r.vv)), 0.5 * (r.hv + from_upper_lane(r.hv))};
+    } else if constexpr (MOM == MOM_V) {
+      const double q = r.vvc / r.hv;
+      r.f[0] = y == NY - 1 ? r.vvc : q;
+      return {r.hv, 0.5 * (r.uu + r.uun), 0.5 * (r.hu + r.hun), 0.5 * (r.vv + r.vvn),
+              0.5 * (r.ho + r.hn)};
+    } else {
+      return {r.ho, r.uu, r.hu, r.vv, r.hv};
+    }
+  };
   auto load_row = [&](int y, Row& r) {
     load_shared(y, r);
 #pragma unroll
@@ -597,16 +649,17 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
     const int fl = (y >= 0 && y < NY) ? (buf.fl & cb.xin) : 0;  // raw masks of the cell
     const int fo = (fl | MB_XOUT) & cb.xm;                      // ... with the column bounds
 
+    const Fields in = fields(y, buf);
     // ---- u/2 on row y: shared part
     const int flm = from_lower_lane(fl), flp = from_upper_lane(fl);
     FaceC<EXACT> fu;
-    face_setup<SCH>(fu, fo & MB_UFLUX, flm & MB_UFLUX, flp & MB_UFLUX, buf.uu, buf.hu, ku,
+    face_setup<SCH>(fu, fo & MB_UFLUX, flm & MB_UFLUX, flp & MB_UFLUX, in.uu, in.hu, ku,
                     dv);
-    const double uum = from_lower_lane(buf.uu);
+    const double uum = from_lower_lane(in.uu);
     const bool updu = fo & MB_UUPD;
-    const double D0 = buf.ho;
+    const double D0 = in.ho;
     double D1 = D0;
-    D1 = sel(updu, D0 - dtu * (buf.uu * dy - uum * dy) * ard1, D0);
+    D1 = sel(updu, D0 - dtu * (in.uu * dy - uum * dy) * ard1, D0);
     CellK k1{};
     Den e1{}, e2{};  // D1, D2 as denominators (EXACT)
     if constexpr (EXACT) e1 = dv.den(D1);
@@ -623,9 +676,9 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
     if constexpr (VF) {
       const bool yface = yv >= isub && yv <= NY - 2 - isub;
       face_setup<SCH>(fv, yface & ((flw[w1] & MB_VFLUX) != 0), flw[w0] & MB_VFLUX,
-                      flw[w2] & MB_VFLUX, buf.vv, buf.hv, kv, dv);
+                      flw[w2] & MB_VFLUX, in.vv, in.hv, kv, dv);
       updv = (yface && yv >= 1 + isub) & ((flw[w1] & MB_VUPD) != 0);
-      D2 = sel(updv, d1w[w1] - dtv * (buf.vv * dx - vvp * dx) * ard1, D2);
+      D2 = sel(updv, d1w[w1] - dtv * (in.vv * dx - vvp * dx) * ard1, D2);
       if constexpr (EXACT) e2 = dv.den(D2);
       else k2 = cell_factors(updv, d1w[w1], D2, dtcv);
     }
@@ -633,7 +686,7 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
     const uint32_t cv = (uint32_t)(x + NX * yv);
     TF res[G];
     double a2v = 0.0;
-    vvp = buf.vv;
+    vvp = in.vv;
     if constexpr (kRowAhead<TF>) load_shared(y + 1, buf);
 
     // u/2 on row y (adv_split_u.F90:219-286)
@@ -733,7 +786,8 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
 // ---- kernel 2: w, then v/2 and u/2 at level K -------------------------------------------
 // BUD: some domain of the launch forms its budgets in the step (the
 // variant without them carries none of their code or registers)
-template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF, bool BUD, typename Div>
+template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF, bool BUD, int MOM,
+          typename Div>
 __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
   StripItem it;
   if (!strip_item<1>(A, it)) return;
@@ -798,8 +852,11 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
   struct Row {
     int fl;
     double wwK, wwKm1, dKm1, dK, dKp1, vv, hv, uu, hu, a2;
+    double wwKn, wwKm1n, ho, hn, uun, hun, vvn, hvn;  // MOM
     TF f[G][5];
   };
+  [[maybe_unused]] const double *ho = MOM ? a.ho + oK : nullptr, *hn = MOM ? a.hn + oK : nullptr;
+  [[maybe_unused]] const uint32_t east = x >= 0 && x + 1 < NX ? 8 : 0;
   auto load_shared = [&](int y, Row& r) {
     const uint32_t c = cell(y), c2 = cell(y - 2);
     const uint32_t b8 = c * 8u, b82 = c2 * 8u;
@@ -810,10 +867,48 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
     r.dK = ldo(dKm1, b8 + lstep);
     r.dKp1 = ldo(dKm1, b8 + lup);
     r.vv = ldo(vv, b82);
-    r.hv = ldo(hv, b82);
     r.uu = ldo(uu, b82);
     r.hu = ldo(hu, b82);
+    if constexpr (MOM == MOM_V) {
+      const uint32_t n = cell(y + 1) * 8u, n2 = cell(y - 1) * 8u;
+      r.wwKn = ldo(wwKm1, n + lstep);
+      r.wwKm1n = ldo(wwKm1, n);
+      r.vvn = ldo(vv, n2);
+      r.uun = ldo(uu, n2);
+      r.hun = ldo(hu, n2);
+      r.ho = ldo(ho, n2);
+      r.hn = ldo(hn, n2);
+    } else {
+      r.hv = ldo(hv, b82);
+      if constexpr (MOM == MOM_U) {
+        r.ho = ldo(ho, b82);
+        r.hn = ldo(hn, b82);
+        // w and v of lane 63 too: the u face of lane 61 reads its tracer
+        r.wwKn = ldo(wwKm1, b8 + lstep + east);
+        r.wwKm1n = ldo(wwKm1, b8 + east);
+        r.vvn = ldo(vv, b82 + east);
+        r.hvn = ldo(hv, b82 + east);
+      }
+    }
     if constexpr (ADV) r.a2 = ldo(a2, b8);
+  };
+  // the row's w, transports and heights (momentum: averaged as in the first
+  // kernel; w at level 0 is zero)
+  struct Fields {
+    double wwK, wwKm1, vv, hv, uu, hu;
+  };
+  auto fields = [&](const Row& r) -> Fields {
+    if constexpr (MOM == MOM_U) {
+      return {0.5 * (r.wwK + r.wwKn), K == 1 ? 0.0 : 0.5 * (r.wwKm1 + r.wwKm1n),
+              0.5 * (r.vv + r.vvn),   0.5 * (r.hv + r.hvn),
+              0.5 * (r.uu + from_upper_lane(r.uu)), from_upper_lane(0.5 * (r.ho + r.hn))};
+    } else if constexpr (MOM == MOM_V) {
+      return {0.5 * (r.wwK + r.wwKn), K == 1 ? 0.0 : 0.5 * (r.wwKm1 + r.wwKm1n),
+              0.5 * (r.vv + r.vvn),   0.5 * (r.ho + r.hn),
+              0.5 * (r.uu + r.uun),   0.5 * (r.hu + r.hun)};
+    } else {
+      return {r.wwK, r.wwKm1, r.vv, r.hv, r.uu, r.hu};
+    }
   };
   auto load_f = [&](int y, Row& r, int g) {
     const uint32_t b = cell(y) * (uint32_t)sizeof(TF);
@@ -865,20 +960,21 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
     const int fl = (y >= 0 && y < NY) ? (buf.fl & cb.xin) : 0;  // raw masks of the cell
     const int fo = (fl | MB_XOUT) & cb.xm;                      // ... with the column bounds
 
+    const Fields in = fields(buf);
     // ---- w on row y: shared part
     const bool wcol = (y <= NY - 2) & ((fo & MB_WCOL) != 0);
     const bool wupd = wcol & kdo;
     const double D2K = buf.dK;
     double D3 = D2K;
-    D3 = sel(wupd, D2K - dt * (buf.wwK - buf.wwKm1), D2K);
+    D3 = sel(wupd, D2K - dt * (in.wwK - in.wwKm1), D2K);
     CellK k3{};
     Den e3{}, e4{}, e5{};  // D3, D4, D5 as denominators (EXACT)
     if constexpr (EXACT) e3 = dv.den(D3);
     else k3 = cell_factors(wupd, D2K, D3, dt);
     WFace<EXACT> wfk, wfp;
     const bool onk = wcol & wk_on, onp = wcol & wp_on;
-    wface_setup<SCH>(wfk, onk ? buf.wwK : 0.0, dt, D2K, buf.dKp1, onk, dv);
-    wface_setup<SCH>(wfp, onp ? buf.wwKm1 : 0.0, dt, buf.dKm1, D2K, onp, dv);
+    wface_setup<SCH>(wfk, onk ? in.wwK : 0.0, dt, D2K, buf.dKp1, onk, dv);
+    wface_setup<SCH>(wfp, onp ? in.wwKm1 : 0.0, dt, buf.dKm1, D2K, onp, dv);
     flw[w3] = fl;
     fow[w3] = fo;
     d3w[w3] = D3;
@@ -892,20 +988,20 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
     if constexpr (VF) {
       const bool yface = yv >= isub && yv <= NY - 2 - isub;
       face_setup<SCH>(fv, yface & ((flw[w1] & MB_VFLUX) != 0), flw[w0] & MB_VFLUX,
-                      flw[w2] & MB_VFLUX, buf.vv, buf.hv, kv, dv);
+                      flw[w2] & MB_VFLUX, in.vv, in.hv, kv, dv);
       updv = (yface && yv >= 1 + isub) & ((flw[w1] & MB_VUPD) != 0);
-      D4 = sel(updv, d3w[w1] - dth * (buf.vv * dx - vvp * dx) * ard1, D4);
+      D4 = sel(updv, d3w[w1] - dth * (in.vv * dx - vvp * dx) * ard1, D4);
       if constexpr (EXACT) e4 = dv.den(D4);
       else k4 = cell_factors(updv, d3w[w1], D4, dtcv);
     }
     if constexpr (VR) {
       const int flv = flw[w1], fov = fow[w1];
       const int flm = from_lower_lane(flv), flp = from_upper_lane(flv);
-      face_setup<SCH>(fu, fov & MB_UFLUX, flm & MB_UFLUX, flp & MB_UFLUX, buf.uu, buf.hu, ku,
+      face_setup<SCH>(fu, fov & MB_UFLUX, flm & MB_UFLUX, flp & MB_UFLUX, in.uu, in.hu, ku,
                     dv);
-      const double uum = from_lower_lane(buf.uu);
+      const double uum = from_lower_lane(in.uu);
       updu = fov & MB_UUPD;
-      D5 = sel(updu, D4 - dth * (buf.uu * dy - uum * dy) * ard1, D4);
+      D5 = sel(updu, D4 - dth * (in.uu * dy - uum * dy) * ard1, D4);
       if constexpr (EXACT) e5 = dv.den(D5);
       else k5 = cell_factors(updu, D4, D5, dtcu);
     }
@@ -913,8 +1009,9 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
     const uint32_t cv = (uint32_t)(x + NX * yv);
     TF res[G], f4[G];
     double a5v = 0.0, a4[ADV ? G : 1];
+    [[maybe_unused]] double fum, fuf;  // MOM: the u fluxes of the row
     [[maybe_unused]] const double A2 = ADV ? buf.a2 : 0.0;
-    vvp = buf.vv;
+    vvp = in.vv;
     if constexpr (kRowAhead<TF>) load_shared(y + 1, buf);
 
     // w on row y (adv_split_w.F90:249-300); a face that does not exist has
@@ -972,7 +1069,10 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
         const TF Fu = face_flux<TF, SCH, DIFF>(fu, fm1, F4, fp1, fp2, AH, ku, dv);
         const TF Fum = from_lower_lane(Fu);
         TF F5 = F4;
-        if constexpr (EXACT) {
+        if constexpr (MOM) {
+          fum = Fum; fuf = Fu;
+          advu = updu ? 0.5 * (Fu * dy - Fum * dy) * ard1 : 0.0;
+        } else if constexpr (EXACT) {
           F5 = cell_update_exact(updu, D4, e5, F4, Fu, Fum, 0.5, dy, ard1, dt, &advu, dv);
         } else {
           F5 = cell_update_fast(k5, F4, Fu, Fum);
@@ -1004,8 +1104,18 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
     }
     // (past the group's last tracer the pointers and values repeat it)
     if (VR && st_ok) {
+      if constexpr (!MOM) {
 #pragma unroll
-      for (int g = 0; g < G; g++) sto(fo_g[g], cv * (uint32_t)sizeof(TF), res[g]);
+        for (int g = 0; g < G; g++) sto(fo_g[g], cv * (uint32_t)sizeof(TF), res[g]);
+      }
+      if constexpr (MOM == MOM_U) {
+        if (yv == NY - 1) {  // the advected velocity the V part starts from there
+          double advn;
+          DivFull df;
+          a.mrow[x + (long)NX * K] = cell_update_exact(updu, D4, df.den(D5), f4[0], fuf, fum, 0.5,
+                                                       dy, ard1, dt, &advn, df);
+        }
+      }
       if constexpr (ADV) {
         if (a.advres) a.advres[oK + cv] = a5v;
       }
@@ -1063,7 +1173,7 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
   if (K == 1 && xout) {
     for (int yv = y0; yv < y0 + A.rows[1] && yv < NY; yv++) {
       const uint32_t c = (uint32_t)(x + NX * yv);
-      for (int g = 0; g < ntr; g++) {
+      for (int g = 0; !MOM && g < ntr; g++) {
         const long tg = (long)(t0 + g) * ts;
         a.fout[tg + c] = a.fin[tg + c];
       }
@@ -1096,34 +1206,36 @@ __device__ __forceinline__ const FusedArgs<TF>& uniform_args(uint64_t p) {
   using Arg = const __attribute__((address_space(4))) FusedArgs<TF>;
   return *(const FusedArgs<TF>*)(Arg*)(((uint64_t)hi << 32) | lo);
 }
-template <typename TF, int SCH, int G, bool ADV, bool DIFF>
+template <typename TF, int SCH, int G, bool ADV, bool DIFF, int MOM>
 __device__ __attribute__((noinline)) void strip_uv_full(uint64_t args) {
   DivFull dv;
-  strip_uv<TF, SCH, G, true, ADV, DIFF>(uniform_args<TF>(args), dv);
+  strip_uv<TF, SCH, G, true, ADV, DIFF, MOM>(uniform_args<TF>(args), dv);
 }
-template <typename TF, int SCH, int G, bool ADV, bool DIFF, bool BUD>
+template <typename TF, int SCH, int G, bool ADV, bool DIFF, bool BUD, int MOM>
 __device__ __attribute__((noinline)) void strip_wvu_full(uint64_t args) {
   DivFull dv;
-  strip_wvu<TF, SCH, G, true, ADV, DIFF, BUD>(uniform_args<TF>(args), dv);
+  strip_wvu<TF, SCH, G, true, ADV, DIFF, BUD, MOM>(uniform_args<TF>(args), dv);
 }
 
-template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF>
+template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF, int MOM = MOM_NONE>
 __global__ __launch_bounds__(256, kWavesUv<TF>) void k_strip_uv(FusedArgs<TF> A) {
   std::conditional_t<EXACT, DivNewton, DivFull> dv;
-  strip_uv<TF, SCH, G, EXACT, ADV, DIFF>(A, dv);
+  strip_uv<TF, SCH, G, EXACT, ADV, DIFF, MOM>(A, dv);
   if constexpr (EXACT) {
     if (dv.bad)
-      strip_uv_full<TF, SCH, G, ADV, DIFF>((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
+      strip_uv_full<TF, SCH, G, ADV, DIFF, MOM>((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
   }
 }
 
-template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF, bool BUD>
+template <typename TF, int SCH, int G, bool EXACT, bool ADV, bool DIFF, bool BUD,
+          int MOM = MOM_NONE>
 __global__ __launch_bounds__(256, kWavesWvu) void k_strip_wvu(FusedArgs<TF> A) {
   std::conditional_t<EXACT, DivNewton, DivFull> dv;
-  strip_wvu<TF, SCH, G, EXACT, ADV, DIFF, BUD>(A, dv);
+  strip_wvu<TF, SCH, G, EXACT, ADV, DIFF, BUD, MOM>(A, dv);
   if constexpr (EXACT) {
     if (dv.bad)
-      strip_wvu_full<TF, SCH, G, ADV, DIFF, BUD>((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
+      strip_wvu_full<TF, SCH, G, ADV, DIFF, BUD, MOM>(
+          (uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
   }
 }
 
@@ -1161,6 +1273,19 @@ hipError_t launch_uv(hipStream_t st, const FusedArgs<TF>& A) {
     default: return hipErrorInvalidValue;
   }
 #undef GT_UV
+  return hipGetLastError();
+}
+
+// both kernels of a momentum variant
+template <int SCH, int MOM>
+hipError_t launch_momentum_one(hipStream_t st, const FusedArgs<double>& A) {
+  auto grid = [&](int p) { return dim3((unsigned)((((A.nitems[p] + 3) / 4 + 7) / 8) * 8)); };
+  hipLaunchKernelGGL((k_strip_uv<double, SCH, 1, true, true, false, MOM>), grid(0), dim3(256), 0,
+                     st, A);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_strip_wvu<double, SCH, 1, true, true, false, false, MOM>), grid(1),
+                     dim3(256), 0, st, A);
   return hipGetLastError();
 }
 

@@ -23,7 +23,9 @@ LIB_NAME = "libgetm_transport.so"
 ORACLE_LIB = "libgetm_oracle.so"
 
 HIP_SOURCES = ["gt_kernels.hip", "gt_api.hip", "gt_batched_f64.hip",
-               "gt_batched_f64_adv.hip", "gt_batched_f64_mom.hip", "gt_batched_f64_g1.hip", "gt_batched_f64_g2.hip",
+               "gt_batched_f64_adv.hip", "gt_batched_f64_mom.hip", "gt_batched_f64_states.hip",
+               "gt_batched_f32_states_g3.hip", "gt_batched_f32_states_g6.hip",
+               "gt_batched_f64_g1.hip", "gt_batched_f64_g2.hip",
                "gt_batched_f32_g1.hip", "gt_batched_f32_g3.hip", "gt_batched_f32_g6.hip",
                "gt_batched_f32_g9.hip",
                "gt_adjoint.hip", "gt_substeps.hip", "gt_eqstate.hip", "gt_inputs.hip",

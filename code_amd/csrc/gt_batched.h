@@ -32,6 +32,8 @@ struct FusedDomain {
   double* d2;         // work: layer heights after u/2 + v/2 (one field)
   double* a2;         // work (ADV): advective term accumulated over u/2 + v/2
   const double *uu, *vv, *ww, *hu, *hv, *ho;
+  // state variants: where f1, f3 and f4 lie, in values from f2 (same layout)
+  long f1_off, f3_off, f4_off;
   const double* hn;      // momentum variants only
   double* mrow;          // work (momentum): the U part's result on the last row, NX per level
   const uint8_t* flags;  // MB_* bits of the mask set of the grid
@@ -86,6 +88,14 @@ hipError_t launch_fused_f32(hipStream_t st, const FusedArgs<float>& a, int group
 // the u and v sub-steps alone, FP64, one tracer: f2, d2 (and a2 with adv)
 // after them (u by fracu*dt, then v by fracv*dt)
 hipError_t launch_strip_uv_f64(hipStream_t st, const FusedArgs<double>& a, bool adv);
+// the HALFSPLIT step with the state after each sub-step kept (f1_off, f2,
+// f3_off, f4_off; fout may be NULL), without budgets; group: states_group's
+hipError_t launch_states_f64(hipStream_t st, const FusedArgs<double>& a);
+hipError_t launch_states_f32(hipStream_t st, const FusedArgs<float>& a, int group);
+template <typename TF>
+constexpr int states_group(int ntracers) {
+  return sizeof(TF) == 8 ? 1 : (ntracers <= 3 ? 3 : 6);
+}
 // the HALFSPLIT step of the velocity on the U (part 0) or V (1) control
 // volumes (uv_advect_3d.F90): advres from uu, vv, ww, ho, hn, hun (as hu) and
 // hvn (as hv); hscheme == vscheme

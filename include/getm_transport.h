@@ -446,7 +446,9 @@ int gt_set_tuning(gt_ctx *ctx, int fused, int tile, int group);
  * 4*c tracer sets instead of 4, and, with per-step inputs, c sets of layer
  * heights instead of one, c = min(ckpt_every, nsteps)); 0 recomputes them per
  * reverse step; -1 (default) keeps them when that needs at most half of the
- * free device memory.  Results are the same bit for bit.  No counterpart in
+ * free device memory, and treats the whole window as one segment
+ * (ckpt_every = nsteps, nothing recomputed) when that needs at most an eighth
+ * of it.  Results are the same bit for bit.  No counterpart in
  * the reference (its reverse mode is this build's extension). */
 int gt_set_adjoint_mode(gt_ctx *ctx, int keep_states);
 /* sizes the context's work fields for the transport step up front (the

@@ -77,6 +77,14 @@ constexpr int kGroup = sizeof(TF) == 8 ? 1 : 6;
 // shorter marches for more wavefronts)
 template <typename TF>
 constexpr int kVRows = sizeof(TF) == 8 ? 8 : 16;
+// most output rows per wavefront of the u and v transposes (marches of 16 and
+// 32 rows recompute six rows each): the launcher halves them where that leaves
+// the chip short of wavefronts.  256 x 256 x 30, one FP64 tracer, 8 / 16 / 24
+// rows: 69 + 62, 57 + 54, 61 + 64 us; 18 FP32 tracers at 320 x 256 x 30,
+// 16 / 32 rows: 351 + 316, 331 + 312 us.
+template <typename TF>
+constexpr int kUVRows = sizeof(TF) == 8 ? 16 : 32;
+constexpr long kUVWaves = 2048;  // ... and how many wavefronts they aim for (2 per SIMD)
 constexpr long kWaveTarget = 8192;  // wavefronts a column march aims for (8 per SIMD)
 constexpr int kUOutF = 60;  // outputs per wavefront of the u forward
 constexpr int kUOutA = 58;  // ... and of the u transpose
@@ -207,21 +215,27 @@ struct RecG {
   T duu, du, dd;
 };
 
+// (Both flavours form every operand and select, as the forward does: returning
+// early for the faces without a limiter cut the marches into blocks in which
+// nothing overlapped.  320 x 256 x 30 x 18 FP32 tracers: w transpose 245 ->
+// 225 us, u and v transposes 364 + 338 -> 351 + 316 us, with fewer registers.)
+
 // the reference arithmetic (reconstruct_bf): rec = fu + (1-cfl)/2 phi(r)
 // deltaf, r = deltafu/deltaf, the branch of phi that the forward's min / max
-// selected; E = 2/(1-cfl) as the face holds it
+// selected; E = 2/(1-cfl) as the face holds it; lim: the limiter applies
 template <int SCH>
-__device__ __forceinline__ RecG<double> rec_grad_exact(double cfl, double E, double fuu, double fu,
-                                                       double fd) {
+__device__ __forceinline__ RecG<double> rec_grad_exact(bool lim, double cfl, double E, double fuu,
+                                                       double fu, double fd) {
   const double g = 0.5 * (1.0 - cfl);
   const double deltaf = fd - fu, deltafu = fu - fuu;
   if constexpr (SCH == UPSTREAM) {
     return {0.0, 1.0, 0.0};
   } else if constexpr (SCH == P2) {  // linear on both branches
     const double x = (1.0 / 6.0) * (1.0 - 2.0 * cfl);
-    return {-g * (0.5 - x), 1.0 - g * (0.5 + x) + g * (0.5 - x), g * (0.5 + x)};
+    return {lim ? -g * (0.5 - x) : 0.0, lim ? 1.0 - g * (0.5 + x) + g * (0.5 - x) : 1.0,
+            lim ? g * (0.5 + x) : 0.0};
   } else {
-    if (!(deltaf * deltafu > 0.0)) return {0.0, 1.0, 0.0};
+    const bool on = lim & (deltaf * deltafu > 0.0);
     const double r = deltafu / deltaf;
     double phi, dphi;
     if constexpr (SCH == P2_PDM) {
@@ -229,67 +243,68 @@ __device__ __forceinline__ RecG<double> rec_grad_exact(double cfl, double E, dou
       const double a = 2.0 * r / (cfl + 1.e-10), b = (0.5 + x) + (0.5 - x) * r;
       const double m = a < b ? a : b;
       const double dm = a < b ? 2.0 / (cfl + 1.e-10) : (0.5 - x);
-      if (E < m) { phi = E; dphi = 0.0; } else { phi = m; dphi = dm; }
+      phi = E < m ? E : m;
+      dphi = E < m ? 0.0 : dm;
     } else if constexpr (SCH == SUPERBEE) {
-      const double a = 2.0 * r < 1.0 ? 2.0 * r : 1.0, da = 2.0 * r < 1.0 ? 2.0 : 0.0;
-      const double b = r < 2.0 ? r : 2.0, db = r < 2.0 ? 1.0 : 0.0;
-      if (a > b) { phi = a; dphi = da; } else { phi = b; dphi = db; }
+      const bool a1 = 2.0 * r < 1.0, b1 = r < 2.0;
+      const double a = a1 ? 2.0 * r : 1.0, da = a1 ? 2.0 : 0.0;
+      const double b = b1 ? r : 2.0, db = b1 ? 1.0 : 0.0;
+      phi = a > b ? a : b;
+      dphi = a > b ? da : db;
     } else {  // MUSCL
       const double a = 2.0 * r, b = 0.5 * (1.0 + r);
       const double m = a < b ? a : b, dm = a < b ? 2.0 : 0.5;
-      if (2.0 < m) { phi = 2.0; dphi = 0.0; } else { phi = m; dphi = dm; }
+      phi = 2.0 < m ? 2.0 : m;
+      dphi = 2.0 < m ? 0.0 : dm;
     }
     // d/dfuu = -g dphi, d/dfu = 1 + g (dphi (1 + r) - phi), d/dfd = g (phi - dphi r)
-    return {-g * dphi, 1.0 + g * (dphi * (1.0 + r) - phi), g * (phi - dphi * r)};
+    return {on ? -g * dphi : 0.0, on ? 1.0 + g * (dphi * (1.0 + r) - phi) : 1.0,
+            on ? g * (phi - dphi * r) : 0.0};
   }
 }
 
 // the FP32 arithmetic (rec_fast): rec = fu + g t, t the branch term the
 // forward's min / max selected, each term linear in du = fu-fuu, df = fd-fu;
-// the identity where the limiter does not apply (g = 0) or deltaf*deltafu <= 0
+// the identity where the limiter does not apply (g = 0) or deltaf*deltafu <=
+// 0.  The terms are compared over the magnitudes, as the forward takes them.
 template <int SCH>
 __device__ __forceinline__ RecG<float> rec_grad_fast(float fuu, float fu, float fd, float g,
                                                      float A, float al, float E) {
   if constexpr (SCH == UPSTREAM) {
     return {0.0f, 1.0f, 0.0f};
   } else {
-    if (g == 0.0f) return {0.0f, 1.0f, 0.0f};
     const float df = fd - fu, du = fu - fuu;
+    bool on = g != 0.0f;
     float tu, tf;  // d t / d du, d t / d df
     if constexpr (SCH == P2) {
       tu = 1.0f - al;
       tf = al;
     } else {
-      if (!(df * du > 0.0f)) return {0.0f, 1.0f, 0.0f};
-      const bool lo = df > 0.0f;  // the min of the terms (else the max)
-      // whether rec_fast's fminf (lo) / fmaxf (hi) of (a, b) returns b
-      auto second = [&](float a, float b) { return lo ? b < a : b > a; };
+      on &= df * du > 0.0f;
+      const float adf = __builtin_fabsf(df), adu = __builtin_fabsf(du);
       if constexpr (SCH == P2_PDM) {
-        const float t1 = A * du, t2 = __builtin_fmaf(al, df - du, du), t3 = E * df;
-        const bool s2 = second(t1, t2);
-        const float m = s2 ? t2 : t1;
-        if (second(m, t3)) { tu = 0.0f; tf = E; }
-        else if (s2) { tu = 1.0f - al; tf = al; }
-        else { tu = A; tf = 0.0f; }
+        const float t1 = A * adu, t2 = __builtin_fmaf(al, adf - adu, adu), t3 = E * adf;
+        const bool s2 = t2 < t1;
+        const bool s3 = t3 < (s2 ? t2 : t1);
+        tu = s3 ? 0.0f : (s2 ? 1.0f - al : A);
+        tf = s3 ? E : (s2 ? al : 0.0f);
       } else if constexpr (SCH == SUPERBEE) {
-        // lo = max(min(2du, df), min(du, 2df)); hi = min(max(2du, df), max(du, 2df))
-        const float a2 = 2.0f * du, b2 = 2.0f * df;
-        const bool inner_a = lo ? (df < a2) : (df > a2);  // first pair: picks df
-        const bool inner_b = lo ? (b2 < du) : (b2 > du);  // second pair: picks 2df
-        const float va = inner_a ? df : a2, vb = inner_b ? b2 : du;
-        const bool outer_b = lo ? (vb > va) : (vb < va);
-        if (outer_b) { tu = inner_b ? 0.0f : 1.0f; tf = inner_b ? 2.0f : 0.0f; }
-        else { tu = inner_a ? 0.0f : 2.0f; tf = inner_a ? 1.0f : 0.0f; }
-      } else {  // MUSCL: lo = min(min(2du, h), 2df), hi = max(...), h = (df+du)/2
-        const float a2 = 2.0f * du, b2 = 2.0f * df, h = 0.5f * (df + du);
-        const bool s2 = second(a2, h);
-        const float m = s2 ? h : a2;
-        if (second(m, b2)) { tu = 0.0f; tf = 2.0f; }
-        else if (s2) { tu = 0.5f; tf = 0.5f; }
-        else { tu = 2.0f; tf = 0.0f; }
+        // max(min(2du, df), min(du, 2df))
+        const float a2 = 2.0f * adu, b2 = 2.0f * adf;
+        const bool inner_a = adf < a2;  // first pair: picks df
+        const bool inner_b = b2 < adu;  // second pair: picks 2df
+        const bool outer_b = (inner_b ? b2 : adu) > (inner_a ? adf : a2);
+        tu = outer_b ? (inner_b ? 0.0f : 1.0f) : (inner_a ? 0.0f : 2.0f);
+        tf = outer_b ? (inner_b ? 2.0f : 0.0f) : (inner_a ? 1.0f : 0.0f);
+      } else {  // MUSCL: min(min(2du, h), 2df), h = (df+du)/2
+        const float a2 = 2.0f * adu, b2 = 2.0f * adf, h = 0.5f * (adf + adu);
+        const bool s2 = h < a2;
+        const bool s3 = b2 < (s2 ? h : a2);
+        tu = s3 ? 0.0f : (s2 ? 0.5f : 2.0f);
+        tf = s3 ? 2.0f : (s2 ? 0.5f : 0.0f);
       }
     }
-    return {-g * tu, 1.0f + g * (tu - tf), g * tf};
+    return {on ? -g * tu : 0.0f, on ? 1.0f + g * (tu - tf) : 1.0f, on ? g * tf : 0.0f};
   }
 }
 
@@ -297,37 +312,33 @@ __device__ __forceinline__ RecG<float> rec_grad_fast(float fuu, float fu, float 
 template <typename TF, int SCH, bool DIFF>
 __device__ __forceinline__ void face_flux_grad(const FaceC<kExact<TF>>& fc, TF fm1, TF f0, TF fp1,
                                                TF fp2, double AH, double dlen, TF out[4]) {
+  RecG<TF> r;
+  bool left;
+  TF vel;  // 0 for a face that carries no flux (not limited either)
   if constexpr (kExact<TF>) {
-    out[0] = out[1] = out[2] = out[3] = 0.0;
-    if (!fc.active) return;
-    const bool left = fc.left, lim = fc.lim;
-    const double fuu = left ? fm1 : fp2, fu0 = left ? f0 : fp1, fd = left ? fp1 : f0;
-    const RecG<double> r =
-        lim ? rec_grad_exact<SCH>(fc.cfl, fc.E, fuu, fu0, fd) : RecG<double>{0.0, 1.0, 0.0};
-    if (left) {
-      out[0] = fc.vel * r.duu; out[1] = fc.vel * r.du; out[2] = fc.vel * r.dd;
-    } else {
-      out[3] = fc.vel * r.duu; out[2] = fc.vel * r.du; out[1] = fc.vel * r.dd;
-    }
-    if constexpr (DIFF) {
-      const double k = AH * fc.Dv / dlen;
-      out[1] += k;
-      out[2] -= k;
-    }
+    left = fc.left;
+    vel = fc.active ? fc.vel : 0.0;
+    r = rec_grad_exact<SCH>(fc.lim, fc.cfl, fc.E, left ? fm1 : fp2, left ? f0 : fp1,
+                            left ? fp1 : f0);
   } else {
-    (void)AH; (void)dlen;
-    const float fuu = fc.right ? fp2 : fm1, fu0 = fc.right ? fp1 : f0, fd = fc.right ? f0 : fp1;
-    const RecG<float> r = rec_grad_fast<SCH>(fuu, fu0, fd, fc.g, fc.A, fc.al, fc.E);
-    if (fc.right) {
-      out[0] = 0.0f; out[1] = fc.vel * r.dd; out[2] = fc.vel * r.du; out[3] = fc.vel * r.duu;
-    } else {
-      out[0] = fc.vel * r.duu; out[1] = fc.vel * r.du; out[2] = fc.vel * r.dd; out[3] = 0.0f;
-    }
-    if constexpr (DIFF) {
-      out[1] += fc.kA;
-      out[2] -= fc.kA;
-    }
+    left = !fc.right;
+    vel = fc.vel;
+    r = rec_grad_fast<SCH>(left ? fm1 : fp2, left ? f0 : fp1, left ? fp1 : f0, fc.g, fc.A, fc.al,
+                           fc.E);
   }
+  const TF duu = vel * r.duu, du = vel * r.du, dd = vel * r.dd;
+  out[0] = left ? duu : TF(0);
+  out[1] = left ? du : dd;
+  out[2] = left ? dd : du;
+  out[3] = left ? TF(0) : duu;
+  if constexpr (DIFF) {
+    TF k;
+    if constexpr (kExact<TF>) k = fc.active ? AH * fc.Dv / dlen : 0.0;
+    else k = fc.kA;
+    out[1] += k;
+    out[2] -= k;
+  }
+  (void)AH; (void)dlen;
 }
 
 // the w flux at face K (K+1/2) from the levels K-1..K+2, and its partials;
@@ -351,16 +362,16 @@ __device__ __forceinline__ void w_flux_grad(const WFace<kExact<TF>>& wf, bool li
   const bool lim = up ? lim_up : lim_dn;
   RecG<TF> r;
   if constexpr (kExact<TF>) {
-    r = lim ? rec_grad_exact<SCH>(wf.cfl, wf.E, fuu, fu, fd) : RecG<double>{0.0, 1.0, 0.0};
+    r = rec_grad_exact<SCH>(lim, wf.cfl, wf.E, fuu, fu, fd);
   } else {
     r = rec_grad_fast<SCH>(fuu, fu, fd, lim ? wf.g : 0.0f, wf.A, wf.al, wf.E);
   }
   const TF w = TF(wf.w);
-  if (up) {
-    out[0] = w * r.duu; out[1] = w * r.du; out[2] = w * r.dd; out[3] = TF(0);
-  } else {
-    out[0] = TF(0); out[1] = w * r.dd; out[2] = w * r.du; out[3] = w * r.duu;
-  }
+  const TF duu = w * r.duu, du = w * r.du, dd = w * r.dd;
+  out[0] = up ? duu : TF(0);
+  out[1] = up ? du : dd;
+  out[2] = up ? dd : du;
+  out[3] = up ? TF(0) : duu;
 }
 
 // ---- the u half sub-step ---------------------------------------------------------
@@ -604,80 +615,53 @@ __global__ __launch_bounds__(256) void k_sub_w(Dims d, int ntr, long ts, const T
   }
 }
 
-// ---- transpose of the u sub-step: one face per lane, cross-lane sums --------
-// Lane L owns cell x and face x (between x and x+1).  Face x reads the cells
-// x-1..x+2 and its flux enters the updates of cells x and x+1; cell x
+// ---- transpose of a u and a v sub-step, in either order: a row march -----------
+// UF: u first (the last two sub-steps of HALFSPLIT, reversed), else v first
+// (the first two).  A wavefront marches the rows of a strip of kUOutA output
+// columns; fu, fv: the states before the u and the v sub-step; lam_in: the
+// adjoint of the later one's output; lam_out: of the earlier one's input.
+//
+// v: the faces Y = y0-2 .. y1 (those of the output rows); before face Y the
+// window holds rows Y-1..Y+2 of the lane's column: each row enters with its
+// diagonal part and mu, collects the terms of the faces whose stencil holds
+// it, and leaves when it is complete (row Y-1 after face Y).
+// u: lane L owns cell x and face x (between x and x+1).  Face x reads the
+// cells x-1..x+2 and its flux enters the updates of cells x and x+1; cell x
 // collects the faces x-2..x+1 (lanes L-2..L+1).  Lanes 3..60 are complete.
-// f: the state before the sub-step; lam_in: the adjoint of its output;
-// lam_out: of its input.
-template <typename TF, int SCH, bool DIFF>
-__global__ __launch_bounds__(256) void k_sub_u_adj(
-    Dims d, int ntr, long ts, const TF* __restrict__ f, const TF* __restrict__ lam_in,
-    TF* __restrict__ lam_out, const double* __restrict__ Dio, const double* __restrict__ Dn,
-    const double* __restrict__ uu, const double* __restrict__ hu,
-    const uint8_t* __restrict__ flags, double dt, double dx, double dy, double ard1, double AH) {
-  constexpr bool EX = kExact<TF>;
-  constexpr int isub = SCH == UPSTREAM ? 0 : 1;
-  const int lane = threadIdx.x;
-  const int x = blockIdx.x * kUOutA - 3 + lane;
-  const int j = blockIdx.y * blockDim.y + threadIdx.y;
-  const int k = blockIdx.z;
-  if (j >= d.NY) return;  // the whole wavefront
-  const bool xin = x >= 0 && x < d.NX;
-  const long c2 = (long)min(max(x, 0), d.NX - 1) + (long)d.NX * j;
-  const long o = d.NXY * (long)k, c = o + c2;
-  const bool out = xin && lane >= 3 && lane <= 60;
-  if (k == 0) {
-    if (out)
-      for (int t = 0; t < ntr; t++) lam_out[t * ts + c] = lam_in[t * ts + c];
-    return;
-  }
-  FaceC<EX> fc = no_face<EX>();
-  if (xin && x <= d.NX - 2)
-    fc = face_at<SCH, EX>(sweep(d, 0), x, c2, o, flags, uu, hu, face_k(0.5 * dt, dx, AH));
-  const bool upd = xin && x >= 1 + isub && x <= d.NX - 2 - isub && (flags[c2] & MB_UUPD);
-  const double fac = 0.5 * dy * ard1;
-  CellOp<EX> cu;
-  if (upd) cu = CellOp<EX>::make(Dio[c], Dn[c], dt * fac);
-  for (int t = 0; t < ntr; t++) {
-    const TF fx = f[t * ts + c], lx = lam_in[t * ts + c];
-    const TF fm1 = from_lower_lane(fx), fp1 = from_upper_lane(fx);
-    const TF fp2 = from_upper_lane(fp1);
-    const TF mu = upd ? cu.mu(lx, dt, fac) : TF(0);  // d(out x)/d F(x) times lam
-    const TF Fbar = mu - from_upper_lane(mu);
-    TF g[4];
-    face_flux_grad<TF, SCH, DIFF>(fc, fm1, fx, fp1, fp2, AH, dx, g);
-    TF acc = upd ? cu.diag(lx) : lx;
-    acc += Fbar * g[1];                                   // face x
-    acc += from_upper_lane(Fbar * g[0]);                  // face x+1
-    acc += from_lower_lane(Fbar * g[2]);                  // face x-1
-    acc += from_lower_lane(from_lower_lane(Fbar * g[3])); // face x-2
-    if (out) lam_out[t * ts + c] = acc;
-  }
-}
-
-// ---- transpose of the v sub-step: a row march -----------------------------------
-// The faces Y = y0-2 .. y1 (those of the output rows); before face Y the
-// window holds rows Y-1..Y+2: each row enters with its diagonal part and mu,
-// collects the terms of the faces whose stencil holds it, and is stored when
-// it leaves (row Y-1 after face Y).
-template <typename TF, int SCH, bool DIFF>
-__global__ __launch_bounds__(64) void k_sub_v_adj(
-    Dims d, int ntr, long ts, const TF* __restrict__ f, const TF* __restrict__ lam_in,
-    TF* __restrict__ lam_out, const double* __restrict__ Dio, const double* __restrict__ Dn,
-    const double* __restrict__ vv, const double* __restrict__ hv,
+// A row passes the u transpose when it enters the window (UF) or when it
+// leaves it, so the adjoint between the two sub-steps stays in registers.
+// The set is read and written once for two sub-steps.  Against a kernel each:
+// 256 x 256 x 30, one FP64 tracer, 28 + 35 -> 59 (u first) and 54 us (v
+// first), bound by the latency of each row's chain; 320 x 256 x 30, 18 FP32
+// tracers, 157 + 223 -> 323 and 312 us, 708 MB each, bound by issue at three
+// wavefronts per SIMD.  The four rows before the first face go through the
+// same loop: unrolled ahead of it they took 60 registers of scratch.
+template <typename TF, int SCH, bool DIFF, bool UF>
+__global__ __launch_bounds__(64, kExact<TF> ? 4 : 3) void k_sub_uv_adj(
+    Dims d, int ntr, long ts, const TF* __restrict__ fu, const TF* __restrict__ fv,
+    const TF* __restrict__ lam_in, TF* __restrict__ lam_out, const double* __restrict__ Du0,
+    const double* __restrict__ Du1, const double* __restrict__ Dv0,
+    const double* __restrict__ Dv1, const double* __restrict__ uu,
+    const double* __restrict__ hu, const double* __restrict__ vv, const double* __restrict__ hv,
     const uint8_t* __restrict__ flags, double dt, double dx, double dy, double ard1, double AH,
-    int ngroups) {
+    int ngroups, int rows) {
   constexpr bool EX = kExact<TF>;
   constexpr int isub = SCH == UPSTREAM ? 0 : 1;
   constexpr int G = kGroup<TF>;
-  const int x = blockIdx.x * 64 + threadIdx.x;
-  const int y0 = blockIdx.y * kVRows<TF>;
+  // whether the u loads of a row are issued a row ahead: where the registers
+  // hold them (FP32, v first: 104 bytes of scratch and 689 us; 12 with
+  // diffusion) and it pays
+  // (FP64, u first: 59 us either way)
+  constexpr bool AHEAD = EX ? !UF : UF && !DIFF;
+  const int lane = threadIdx.x;
+  const int x = blockIdx.x * kUOutA - 3 + lane;
+  const int y0 = blockIdx.y * rows;
   const int k = blockIdx.z / ngroups, t0 = (blockIdx.z % ngroups) * G;
-  if (x >= d.NX) return;  // no cross-lane moves here
   const int NX = d.NX, NY = d.NY;
+  const bool xin = x >= 0 && x < NX, out = xin && lane >= 3 && lane <= 60;
+  const int xc = min(max(x, 0), NX - 1);
   const long o = d.NXY * (long)k;
-  const int y1 = min(y0 + kVRows<TF>, NY);
+  const int y1 = min(y0 + rows, NY);
   long tb[G];
 #pragma unroll
   for (int g = 0; g < G; g++) tb[g] = (long)min(t0 + g, ntr - 1) * ts;
@@ -685,75 +669,141 @@ __global__ __launch_bounds__(64) void k_sub_v_adj(
     for (int y = y0; y < y1; y++)
 #pragma unroll
       for (int g = 0; g < G; g++)
-        if (t0 + g < ntr) lam_out[tb[g] + x + (long)NX * y] = lam_in[tb[g] + x + (long)NX * y];
+        if (out && t0 + g < ntr) lam_out[tb[g] + x + (long)NX * y] = lam_in[tb[g] + x + (long)NX * y];
     return;
   }
-  const FaceK fk = face_k(0.5 * dt, dy, AH);
-  const double fac = 0.5 * dx * ard1;
+  const FaceK fku = face_k(0.5 * dt, dx, AH), fkv = face_k(0.5 * dt, dy, AH);
+  const double facu = 0.5 * dy * ard1, facv = 0.5 * dx * ard1;
+  auto row_of = [&](int y) -> long { return o + xc + (long)NX * (y >= 0 && y < NY ? y : 0); };
+
+  // the u transpose of row y: its loads, and l -> its adjoint in place
+  struct URaw {
+    TF f[G];
+    double D0, D1, vel, Dv;
+    uint8_t fm, fc, fp;
+  };
+  auto fetch_u = [&](int y) -> URaw {
+    const long c = row_of(y);
+    URaw r;
+    r.D0 = Du0[c];
+    r.D1 = Du1[c];
+    r.vel = uu[c];
+    r.Dv = hu[c];
+    r.fc = flags[c - o];
+    r.fm = flags[c - o - (xc > 0)];
+    r.fp = flags[c - o + (xc < NX - 1)];
+#pragma unroll
+    for (int g = 0; g < G; g++) r.f[g] = fu[tb[g] + c];
+    return r;
+  };
+  auto u_adj = [&](const URaw& r, TF (&l)[G]) {
+    FaceC<EX> fc = no_face<EX>();
+    if (xin && x <= NX - 2) {
+      const bool active = x >= isub && x <= NX - 2 - isub && (r.fc & MB_UFLUX);
+      const bool lim_l = SCH != UPSTREAM && x >= 1 && (r.fm & MB_UFLUX);
+      const bool lim_r = SCH != UPSTREAM && (r.fp & MB_UFLUX);
+      DivFull dv;
+      face_setup<SCH>(fc, active, lim_l, lim_r, r.vel, r.Dv, fku, dv);
+    }
+    const bool upd = xin && x >= 1 + isub && x <= NX - 2 - isub && (r.fc & MB_UUPD);
+    CellOp<EX> cu;
+    if (upd) cu = CellOp<EX>::make(r.D0, r.D1, dt * facu);
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      const TF fx = r.f[g], lx = l[g];
+      const TF fm1 = from_lower_lane(fx), fp1 = from_upper_lane(fx);
+      const TF fp2 = from_upper_lane(fp1);
+      const TF mu = upd ? cu.mu(lx, dt, facu) : TF(0);  // d(out x)/d F(x) times lam
+      const TF Fbar = mu - from_upper_lane(mu);
+      TF q[4];
+      face_flux_grad<TF, SCH, DIFF>(fc, fm1, fx, fp1, fp2, AH, dx, q);
+      TF acc = upd ? cu.diag(lx) : lx;
+      acc += Fbar * q[1];                                   // face x
+      acc += from_upper_lane(Fbar * q[0]);                  // face x+1
+      acc += from_lower_lane(Fbar * q[2]);                  // face x-1
+      acc += from_lower_lane(from_lower_lane(Fbar * q[3])); // face x-2
+      l[g] = acc;
+    }
+  };
+
   struct Row {
     TF f, acc, mu;
   };
-  Row w[G][4];
+  Row w[G][4] = {};
   // the loads of a row entering the window, read one face ahead
   struct ERaw {
     TF l[G], f[G];
-    double Dio, Dn;
+    double D0, D1;
     uint8_t fl;
   };
   auto fetch = [&](int y) -> ERaw {
-    const bool yin = y >= 0 && y < NY;
-    const long cy = o + x + (long)NX * (yin ? y : 0);
+    const long c = row_of(y);
     ERaw r;
-    r.Dio = Dio[cy];
-    r.Dn = Dn[cy];
-    r.fl = flags[cy - o];
+    r.D0 = Dv0[c];
+    r.D1 = Dv1[c];
+    r.fl = flags[c - o];
 #pragma unroll
     for (int g = 0; g < G; g++) {
-      r.l[g] = lam_in[tb[g] + cy];
-      r.f[g] = f[tb[g] + cy];
+      r.l[g] = lam_in[tb[g] + c];
+      r.f[g] = fv[tb[g] + c];
     }
     return r;
   };
-  // row y enters the window slot q
-  auto enter = [&](int y, int q, const ERaw& r) {
-    const bool yin = y >= 0 && y < NY;
+  // row y enters the window (UF: through its u transpose)
+  auto enter = [&](int y, ERaw r, const URaw& ur) {
+    if constexpr (UF) u_adj(ur, r.l);
+    const bool yin = xin && y >= 0 && y < NY;
     const bool upd = yin && y >= 1 + isub && y <= NY - 2 - isub && (r.fl & MB_VUPD);
     CellOp<EX> cu;
-    if (upd) cu = CellOp<EX>::make(r.Dio, r.Dn, dt * fac);
+    if (upd) cu = CellOp<EX>::make(r.D0, r.D1, dt * facv);
 #pragma unroll
     for (int g = 0; g < G; g++) {
       const TF l = r.l[g];
-      w[g][q].f = r.f[g];
-      w[g][q].acc = upd ? cu.diag(l) : l;
-      w[g][q].mu = upd ? cu.mu(l, dt, fac) : TF(0);
+      w[g][3].f = r.f[g];
+      w[g][3].acc = upd ? cu.diag(l) : l;
+      w[g][3].mu = upd ? cu.mu(l, dt, facv) : TF(0);
     }
   };
-  enter(y0 - 3, 0, fetch(y0 - 3));
-  enter(y0 - 2, 1, fetch(y0 - 2));
-  enter(y0 - 1, 2, fetch(y0 - 1));
-  enter(y0, 3, fetch(y0));
-  ERaw en = fetch(y0 + 1);
-  VRaw rn = vraw(d, x, o, y0 - 2, flags, vv, hv, Dio, Dn);
-  for (int Y = y0 - 2; Y <= y1; Y++) {
-    const VRaw r = rn;
-    rn = vraw(d, x, o, Y + 1, flags, vv, hv, Dio, Dn);
+  // four rows enter before the first face
+  ERaw en = fetch(y0 - 3);
+  URaw un{};  // UF: of the next row to enter; else of the next to leave
+  if constexpr (AHEAD) un = fetch_u(UF ? y0 - 3 : y0);
+  VRaw rn = vraw(d, xc, o, y0 - 2, flags, vv, hv, Dv0, Dv1);
+  for (int Y = y0 - 6; Y <= y1; Y++) {
     const ERaw e = en;
     en = fetch(Y + 4);
-    FaceC<EX> fc = no_face<EX>();
-    if (Y >= 0 && Y <= NY - 2) fc = vface<SCH, EX>(d, Y, r, fk);
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-      const TF Fbar = w[g][1].mu - w[g][2].mu;
-      TF gr[4];
-      face_flux_grad<TF, SCH, DIFF>(fc, w[g][0].f, w[g][1].f, w[g][2].f, w[g][3].f, AH, dy, gr);
-#pragma unroll
-      for (int q = 0; q < 4; q++) w[g][q].acc += Fbar * gr[q];
+    URaw ur = un;
+    if constexpr (UF) {
+      if constexpr (AHEAD) un = fetch_u(Y + 4);
+      else ur = fetch_u(Y + 3);
     }
-    const int yd = Y - 1;  // complete
-    if (yd >= y0 && yd < y1) {
+    if (Y >= y0 - 2) {
+      const VRaw r = rn;
+      rn = vraw(d, xc, o, Y + 1, flags, vv, hv, Dv0, Dv1);
+      FaceC<EX> fc = no_face<EX>();
+      if (Y >= 0 && Y <= NY - 2) fc = vface<SCH, EX>(d, Y, r, fkv);
 #pragma unroll
-      for (int g = 0; g < G; g++)
-        if (t0 + g < ntr) lam_out[tb[g] + o + x + (long)NX * yd] = w[g][0].acc;
+      for (int g = 0; g < G; g++) {
+        const TF Fbar = w[g][1].mu - w[g][2].mu;
+        TF gr[4];
+        face_flux_grad<TF, SCH, DIFF>(fc, w[g][0].f, w[g][1].f, w[g][2].f, w[g][3].f, AH, dy, gr);
+#pragma unroll
+        for (int q = 0; q < 4; q++) w[g][q].acc += Fbar * gr[q];
+      }
+      const int yd = Y - 1;  // complete
+      if (yd >= y0 && yd < y1) {
+        TF l[G];
+#pragma unroll
+        for (int g = 0; g < G; g++) l[g] = w[g][0].acc;
+        if constexpr (!UF) {
+          if constexpr (AHEAD) un = fetch_u(yd + 1);
+          else ur = fetch_u(yd);
+          u_adj(ur, l);
+        }
+#pragma unroll
+        for (int g = 0; g < G; g++)
+          if (out && t0 + g < ntr) lam_out[tb[g] + o + x + (long)NX * yd] = l[g];
+      }
     }
 #pragma unroll
     for (int g = 0; g < G; g++) {
@@ -761,7 +811,7 @@ __global__ __launch_bounds__(64) void k_sub_v_adj(
       w[g][1] = w[g][2];
       w[g][2] = w[g][3];
     }
-    enter(Y + 3, 3, e);
+    enter(Y + 3, e, ur);
   }
 }
 
@@ -934,56 +984,56 @@ hipError_t launch_heights(hipStream_t st, Dims d, const uint8_t* flags, const do
   return hipGetLastError();
 }
 
-// ADJ: a = f, b = lam_in, out = lam_out; else a = fin, out = fout
-template <typename TF, bool ADJ, int SCH, bool DIFF>
-static void launch_h_one(hipStream_t st, Dims d, int dir, int ntr, long ts, const TF* a,
-                         const TF* b, TF* out, const double* Dio, const double* Dn,
-                         const double* vel, const double* Dv, const uint8_t* flags, double dt,
-                         double dx, double dy, double ard1, double AH) {
+// f(scheme, diffusion) with both as compile-time constants
+#define GT_H(S) (AH > 0.0 ? GT_H1(S, true) : GT_H1(S, false))
+#define GT_H_SCHEMES()                        \
+  switch (scheme) {                           \
+    case UPSTREAM: GT_H(UPSTREAM); break;     \
+    case P2: GT_H(P2); break;                 \
+    case SUPERBEE: GT_H(SUPERBEE); break;     \
+    case MUSCL: GT_H(MUSCL); break;           \
+    case P2_PDM: GT_H(P2_PDM); break;         \
+    default: return hipErrorInvalidValue;     \
+  }                                           \
+  return hipGetLastError()
+
+template <typename TF, int SCH, bool DIFF>
+static void launch_h_one(hipStream_t st, Dims d, int dir, int ntr, long ts, const TF* fin,
+                         TF* fout, const double* Dio, const double* Dn, const double* vel,
+                         const double* Dv, const uint8_t* flags, double dt, double dx, double dy,
+                         double ard1, double AH) {
   const int ng = (ntr + kGroup<TF> - 1) / kGroup<TF>;
   const dim3 gv((d.NX + 63) / 64, (d.NY + kVRows<TF> - 1) / kVRows<TF>, (d.kmax + 1) * ng);
-  if constexpr (ADJ) {
-    if (dir == 0)
-      hipLaunchKernelGGL((k_sub_u_adj<TF, SCH, DIFF>),
-                         dim3((d.NX + kUOutA - 1) / kUOutA, (d.NY + 3) / 4, d.kmax + 1),
-                         dim3(64, 4), 0, st, d, ntr, ts, a, b, out, Dio, Dn, vel, Dv, flags, dt,
-                         dx, dy, ard1, AH);
-    else
-      hipLaunchKernelGGL((k_sub_v_adj<TF, SCH, DIFF>), gv, dim3(64), 0, st, d, ntr, ts, a, b, out,
-                         Dio, Dn, vel, Dv, flags, dt, dx, dy, ard1, AH, ng);
-  } else {
-    (void)b;
-    if (dir == 0)
-      hipLaunchKernelGGL((k_sub_u<TF, SCH, DIFF>),
-                         dim3((d.NX + kUOutF - 1) / kUOutF, (d.NY + 3) / 4, d.kmax + 1),
-                         dim3(64, 4), 0, st, d, ntr, ts, a, out, Dio, Dn, vel, Dv, flags, dt, dx,
-                         dy, ard1, AH);
-    else
-      hipLaunchKernelGGL((k_sub_v<TF, SCH, DIFF>), gv, dim3(64), 0, st, d, ntr, ts, a, out, Dio,
-                         Dn, vel, Dv, flags, dt, dx, dy, ard1, AH, ng);
-  }
+  if (dir == 0)
+    hipLaunchKernelGGL((k_sub_u<TF, SCH, DIFF>),
+                       dim3((d.NX + kUOutF - 1) / kUOutF, (d.NY + 3) / 4, d.kmax + 1),
+                       dim3(64, 4), 0, st, d, ntr, ts, fin, fout, Dio, Dn, vel, Dv, flags, dt, dx,
+                       dy, ard1, AH);
+  else
+    hipLaunchKernelGGL((k_sub_v<TF, SCH, DIFF>), gv, dim3(64), 0, st, d, ntr, ts, fin, fout, Dio,
+                       Dn, vel, Dv, flags, dt, dx, dy, ard1, AH, ng);
 }
 
-template <typename TF, bool ADJ>
-static hipError_t launch_h(hipStream_t st, Dims d, int dir, int ntr, long ts, const TF* a,
-                           const TF* b, TF* out, const double* Dio, const double* Dn,
-                           const double* vel, const double* Dv, const uint8_t* flags, double dt,
-                           double dx, double dy, double ard1, int scheme, double AH) {
-#define GT_H(S)                                                                                \
-  (AH > 0.0 ? launch_h_one<TF, ADJ, S, true>(st, d, dir, ntr, ts, a, b, out, Dio, Dn, vel, Dv,  \
-                                             flags, dt, dx, dy, ard1, AH)                      \
-            : launch_h_one<TF, ADJ, S, false>(st, d, dir, ntr, ts, a, b, out, Dio, Dn, vel, Dv, \
-                                              flags, dt, dx, dy, ard1, AH))
-  switch (scheme) {
-    case UPSTREAM: GT_H(UPSTREAM); break;
-    case P2: GT_H(P2); break;
-    case SUPERBEE: GT_H(SUPERBEE); break;
-    case MUSCL: GT_H(MUSCL); break;
-    case P2_PDM: GT_H(P2_PDM); break;
-    default: return hipErrorInvalidValue;
-  }
-#undef GT_H
-  return hipGetLastError();
+template <typename TF, int SCH, bool DIFF>
+static void launch_uv_adj_one(hipStream_t st, Dims d, bool ufirst, int ntr, long ts, const TF* fu,
+                              const TF* fv, const TF* lam_in, TF* lam_out, const double* Du0,
+                              const double* Du1, const double* Dv0, const double* Dv1,
+                              const double* uu, const double* hu, const double* vv,
+                              const double* hv, const uint8_t* flags, double dt, double dx,
+                              double dy, double ard1, double AH) {
+  const int ng = (ntr + kGroup<TF> - 1) / kGroup<TF>;
+  const int nsx = (d.NX + kUOutA - 1) / kUOutA;
+  int rows = kUVRows<TF>;
+  while (rows > 4 && (long)nsx * ((d.NY + rows - 1) / rows) * d.kmax * ng < kUVWaves) rows /= 2;
+  const dim3 g(nsx, (d.NY + rows - 1) / rows, (d.kmax + 1) * ng);
+  if (ufirst)
+    hipLaunchKernelGGL((k_sub_uv_adj<TF, SCH, DIFF, true>), g, dim3(64), 0, st, d, ntr, ts, fu,
+                       fv, lam_in, lam_out, Du0, Du1, Dv0, Dv1, uu, hu, vv, hv, flags, dt, dx, dy,
+                       ard1, AH, ng, rows);
+  else
+    hipLaunchKernelGGL((k_sub_uv_adj<TF, SCH, DIFF, false>), g, dim3(64), 0, st, d, ntr, ts, fu,
+                       fv, lam_in, lam_out, Du0, Du1, Dv0, Dv1, uu, hu, vv, hv, flags, dt, dx, dy,
+                       ard1, AH, ng, rows);
 }
 
 template <typename TF, bool ADJ, int SCH>
@@ -1031,18 +1081,28 @@ hipError_t launch_sub_h(hipStream_t st, Dims d, int dir, int ntr, long ts, const
                         const double* Dio, const double* Dn, const double* vel, const double* Dv,
                         const uint8_t* flags, double dt, double dx, double dy, double ard1,
                         int scheme, double AH) {
-  return launch_h<TF, false>(st, d, dir, ntr, ts, fin, nullptr, fout, Dio, Dn, vel, Dv, flags, dt,
-                             dx, dy, ard1, scheme, AH);
+#define GT_H1(S, DF)                                                                          \
+  launch_h_one<TF, S, DF>(st, d, dir, ntr, ts, fin, fout, Dio, Dn, vel, Dv, flags, dt, dx, dy, \
+                          ard1, AH)
+  GT_H_SCHEMES();
+#undef GT_H1
 }
 
 template <typename TF>
-hipError_t launch_sub_h_adj(hipStream_t st, Dims d, int dir, int ntr, long ts, const TF* f,
-                            const TF* lam_in, TF* lam_out, const double* Dio, const double* Dn,
-                            const double* vel, const double* Dv, const uint8_t* flags, double dt,
-                            double dx, double dy, double ard1, int scheme, double AH) {
-  return launch_h<TF, true>(st, d, dir, ntr, ts, f, lam_in, lam_out, Dio, Dn, vel, Dv, flags, dt,
-                            dx, dy, ard1, scheme, AH);
+hipError_t launch_sub_uv_adj(hipStream_t st, Dims d, bool ufirst, int ntr, long ts, const TF* fu,
+                             const TF* fv, const TF* lam_in, TF* lam_out, const double* Du0,
+                             const double* Du1, const double* Dv0, const double* Dv1,
+                             const double* uu, const double* hu, const double* vv,
+                             const double* hv, const uint8_t* flags, double dt, double dx,
+                             double dy, double ard1, int scheme, double AH) {
+#define GT_H1(S, DF)                                                                            \
+  launch_uv_adj_one<TF, S, DF>(st, d, ufirst, ntr, ts, fu, fv, lam_in, lam_out, Du0, Du1, Dv0,  \
+                               Dv1, uu, hu, vv, hv, flags, dt, dx, dy, ard1, AH)
+  GT_H_SCHEMES();
+#undef GT_H1
 }
+#undef GT_H
+#undef GT_H_SCHEMES
 
 template <typename TF>
 hipError_t launch_sub_w(hipStream_t st, Dims d, int ntr, long ts, const TF* fin, TF* fout,
@@ -1066,10 +1126,11 @@ hipError_t launch_sub_w_adj(hipStream_t st, Dims d, int ntr, long ts, const TF* 
                                        const double*, const double*, const double*,            \
                                        const double*, const uint8_t*, double, double, double,  \
                                        double, int, double);                                   \
-  template hipError_t launch_sub_h_adj<TF>(hipStream_t, Dims, int, int, long, const TF*,       \
-                                           const TF*, TF*, const double*, const double*,       \
-                                           const double*, const double*, const uint8_t*,       \
-                                           double, double, double, double, int, double);       \
+  template hipError_t launch_sub_uv_adj<TF>(                                                   \
+      hipStream_t, Dims, bool, int, long, const TF*, const TF*, const TF*, TF*, const double*, \
+      const double*, const double*, const double*, const double*, const double*,               \
+      const double*, const double*, const uint8_t*, double, double, double, double, int,       \
+      double);                                                                                 \
   template hipError_t launch_sub_w<TF>(hipStream_t, Dims, int, long, const TF*, TF*,           \
                                        const double*, const double*, const double*,            \
                                        const uint8_t*, double, int, int);                      \

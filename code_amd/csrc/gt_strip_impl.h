@@ -64,7 +64,11 @@ __device__ __forceinline__ double rcp_nr(double x) {
 // a tiny numerator (below ~2^-969) leaves it denormal; an infinity, a NaN, a
 // zero or denormal b or an overflow leaves it infinite or NaN.  DivNewton
 // collects that test over the lanes whose quotient is used, and a strip in
-// which it fired is marched again with DivFull.  (A zero numerator gives +0
+// which it fired is given up there (asked after the first row, the fourth and
+// every four) and marched again with DivFull: tails of a tracer that fade out
+// below 1e-292 reach it, and a field that lies there as a whole (400 x 400 x
+// 40, two tracers: 480 us) would take 775 with the strips marched to their
+// end first.  (A zero numerator gives +0
 // where the full sequence keeps its sign.  |b| stays below 2^1021.)
 struct Den {
   double b, y;
@@ -74,6 +78,7 @@ struct DivFull {
   __device__ __forceinline__ double over(double a, const Den& d, bool) const { return a / d.b; }
   __device__ __forceinline__ double div(double a, double b, bool) const { return a / b; }
   __device__ __forceinline__ void pin() const {}
+  __device__ __forceinline__ bool stop() const { return false; }
 };
 struct DivNewton {
   uint64_t bad = 0;    // the lanes it fired on, up to the last pin()
@@ -103,6 +108,7 @@ struct DivNewton {
     asm volatile("" : "+s"(bad));
     fired = false;
   }
+  __device__ __forceinline__ bool stop() const { return bad != 0; }
 };
 
 // ---- one face of a sweep -----------------------------------------------------
@@ -772,14 +778,17 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
   Row r;
   if constexpr (kRowAhead<TF>) load_row(y0 - 2, r);
   step(Slot<0>{}, off, off, r, 0);
+  if (dv.stop()) return;
   step(Slot<1>{}, off, off, r, 1);
   step(Slot<2>{}, off, off, r, 2);
   step(Slot<3>{}, on, off, r, 3);
+  if (dv.stop()) return;
   for (int s = 4; s < nsteps; s += 4) {
     step(Slot<0>{}, on, on, r, s);
     step(Slot<1>{}, on, on, r, s + 1);
     step(Slot<2>{}, on, on, r, s + 2);
     step(Slot<3>{}, on, on, r, s + 3);
+    if (dv.stop()) return;
   }
 
   // level 0 of the work fields (the second kernel reads levels K-2..K+2 of
@@ -1159,14 +1168,17 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
   Row r;
   if constexpr (kRowAhead<TF>) load_row(y0 - 2, r);
   step(Slot<0>{}, off, off, r, 0);
+  if (dv.stop()) return;
   step(Slot<1>{}, off, off, r, 1);
   step(Slot<2>{}, off, off, r, 2);
   step(Slot<3>{}, on, off, r, 3);
+  if (dv.stop()) return;
   for (int s = 4; s < nsteps; s += 4) {
     step(Slot<0>{}, on, on, r, s);
     step(Slot<1>{}, on, on, r, s + 1);
     step(Slot<2>{}, on, on, r, s + 2);
     step(Slot<3>{}, on, on, r, s + 3);
+    if (dv.stop()) return;
   }
 
   // the budget partials of this strip-level: the lanes' sums added over the

@@ -480,11 +480,12 @@ int gt_autotune_batch(int ndom, const gt_batch_domain *doms, int ntracers,
  * lam0 = (d f_final / d f0)^T lam_final.  The limiter enters through the
  * derivative of the branch the forward took.  The reverse sweep recomputes
  * each segment from its checkpoint and applies the transpose of each
- * sub-step; the states before the sub-steps come from the per-sub-step
- * kernels (bit-identical to the strip kernels), kept for the whole segment
- * or recomputed per reverse step (gt_set_adjoint_mode).  Work memory in FP64
- * fields, with c = min(ckpt_every, nsteps): 5 + 2 + ceil(nsteps/ckpt_every)
- * + c - 1, plus 4 (states recomputed) or 4*c (states kept). */
+ * sub-step; the states before the sub-steps come from the strip kernels
+ * (from the per-sub-step kernels, bit-identical to them, where those do not
+ * apply), kept for the whole segment or recomputed per reverse step
+ * (gt_set_adjoint_mode).  Work memory in FP64 fields, with c =
+ * min(ckpt_every, nsteps), or nsteps where the window is one segment: 5 + 2 +
+ * ceil(nsteps/c) + c - 1, plus 4 (states recomputed) or 4*c (states kept). */
 int gt_adv3d_adjoint(gt_ctx *ctx, int nsteps, int ckpt_every, double dt,
                      const double *f0, double *f_final, const double *lam_final,
                      double *lam0, const double *uu, const double *vv,
@@ -499,9 +500,9 @@ int gt_adv3d_adjoint(gt_ctx *ctx, int nsteps, int ckpt_every, double dt,
  * reverse sweep recomputes each step's sub-step states from the checkpoint
  * (kept per segment or per reverse step, gt_set_adjoint_mode) and applies
  * the transpose of each FP32 sub-step, the limiter through the derivative of
- * the branch term the FP32 forward selected.  Work memory, with c =
- * min(ckpt_every, nsteps): 5 FP64 fields + (2 + ceil(nsteps/ckpt_every) +
- * c - 1 + 4 or 4*c) tracer sets of ntracers FP32 fields. */
+ * the branch term the FP32 forward selected.  Work memory, c as above: 5
+ * FP64 fields + (2 + ceil(nsteps/c) + c - 1 + 4 or 4*c) tracer sets of
+ * ntracers FP32 fields. */
 int gt_adv3d_adjoint_f32(gt_ctx *ctx, int ntracers, int nsteps, int ckpt_every,
                          double dt, const float *f0, float *f_final,
                          const float *lam_final, float *lam0, const double *uu,

@@ -59,30 +59,51 @@ __device__ __forceinline__ double rcp_nr(double x) {
 // pass their operands through, so the Newton steps and the last three
 // operations alone give the same bits, and y is formed once for every
 // quotient over the same b (the cell updates of the tracers, P2-PDM's
-// 2r/(cfl+1e-10), the division by dx).  What scaling guards against shows in
-// the remainder r, which is exact for a normal quotient of normal operands:
-// a tiny numerator (below ~2^-969) leaves it denormal; an infinity, a NaN, a
-// zero or denormal b or an overflow leaves it infinite or NaN.  DivNewton
-// collects that test over the lanes whose quotient is used, and a strip in
-// which it fired is given up there (asked after the first row, the fourth and
-// every four) and marched again with DivFull: tails of a tracer that fade out
-// below 1e-292 reach it, and a field that lies there as a whole (400 x 400 x
-// 40, two tracers: 480 us) would take 775 with the strips marched to their
-// end first.  (A zero numerator gives +0
-// where the full sequence keeps its sign.  |b| stays below 2^1021.)
+// 2r/(cfl+1e-10), the division by dx).  They need a remainder that is exact
+// and a quotient that is normal; DivNewton tests for what takes that away and
+// gives a strip up where it fires (asked after the first row, the fourth and
+// every four), which is then marched again with DivFull:
+//   * a numerator below 2^-969, zero aside: its remainder ends in the
+//     denormals, rounded, or flushed to a zero that looks exact (a < 2^-1021
+//     over |b| < 1);
+//   * an infinity, a NaN, a zero b or an overflow (q infinite or NaN), and a
+//     denormal q (rounded twice).
+// What is known of a quotient (Quot) saves part of the test.  Not covered: |b|
+// of 2^1022 or more, Courant numbers beyond 2^50, and a quotient within one
+// rounding of 2^-1075.
+// A zero numerator gives +0 where the full sequence keeps its sign.
+// Cost and reach (400 x 400 x 40, two tracers, P2-PDM): 380 us where nothing
+// fires (375 with the remainder's class as the only test, 470 with full
+// divisions alone); tails of a tracer that fade out below 1e-292 fire it: a
+// patch in an empty basin after 30 / 300 steps 400 / 432 us (441 / 450), a
+// field that lies there as a whole 462 (469).
 struct Den {
   double b, y;
 };
+// what is known of a quotient.  kNonzero: its numerator is not zero where it is
+// used.  kFace: a Courant number, whose last bits vanish in 1 - c, 1 - 2c and
+// c + 1e-10 where it is tiny.  kRatio: twice a tested quotient on top, so a
+// numerator of 2^-1021 or more, whose remainder tells the rest (one that rounds
+// to zero leaves q0 the nearest).  kBound: P2-PDM's 2/(1-c), tested with c, and
+// NaN for c = 1, which the min takes for the infinity it stands for.
+enum Quot { kAny, kNonzero, kFace, kRatio, kBound };
 struct DivFull {
   __device__ __forceinline__ Den den(double b) const { return {b, 0.0}; }
-  __device__ __forceinline__ double over(double a, const Den& d, bool) const { return a / d.b; }
-  __device__ __forceinline__ double div(double a, double b, bool) const { return a / b; }
+  template <Quot Q = kAny>
+  __device__ __forceinline__ double over(double a, const Den& d, bool) const {
+    return a / d.b;
+  }
+  template <Quot Q = kAny>
+  __device__ __forceinline__ double div(double a, double b, bool) const {
+    return a / b;
+  }
   __device__ __forceinline__ void pin() const {}
   __device__ __forceinline__ bool stop() const { return false; }
 };
 struct DivNewton {
   uint64_t bad = 0;    // the lanes it fired on, up to the last pin()
   bool fired = false;  // and since
+  static constexpr uint32_t kLow = (1023 - 969) << 21;  // 2^-969's bits past the sign
   __device__ __forceinline__ Den den(double b) const {
     double y = __builtin_amdgcn_rcp(b);
     y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
@@ -90,17 +111,28 @@ struct DivNewton {
     return {b, y};
   }
   // a/b; used: whether this lane's quotient reaches a result
+  template <Quot Q = kAny>
   __device__ __forceinline__ double over(double a, const Den& d, bool used) {
     constexpr int kNanInfDenorm = 0x1 | 0x2 | 0x4 | 0x10 | 0x80 | 0x200;
     const double q0 = a * d.y;
     const double r = __builtin_fma(-d.b, q0, a);
-    fired |= used & __builtin_amdgcn_class(r, kNanInfDenorm);
-    return __builtin_fma(r, d.y, q0);
+    const double q = __builtin_fma(r, d.y, q0);
+    if constexpr (Q == kNonzero) {
+      fired |= used & ((__builtin_fabs(a) < 0x1p-969) | __builtin_amdgcn_class(q, kNanInfDenorm));
+    } else if constexpr (Q == kAny) {
+      // the bits past the sign, less one: a zero comes out largest
+      const uint64_t m = (__builtin_bit_cast(uint64_t, a) << 1) - 1;
+      fired |= used & (((uint32_t)(m >> 32) < kLow) | __builtin_amdgcn_class(q, kNanInfDenorm));
+    } else if constexpr (Q != kBound) {
+      fired |= used & __builtin_amdgcn_class(r, kNanInfDenorm);
+    }
+    return q;
   }
+  template <Quot Q = kAny>
   __device__ __forceinline__ double div(double a, double b, bool used) {
-    return over(a, den(b), used);
+    return over<Q>(a, den(b), used);
   }
-  // ends a section of the row: the tests of the section's remainders stay in
+  // ends a section of the row: the tests of the section's quotients stay in
   // it (left to the compiler they gather at the row's end and keep every
   // remainder in registers until there)
   __device__ __forceinline__ void pin() {
@@ -158,10 +190,11 @@ __device__ __forceinline__ void face_setup(FaceC<true>& fc, bool active, bool li
   fc.active = active;
   fc.left = left;
   fc.lim = lim;
-  const double c = dv.over(dv.div(left ? vel : -vel, Dv, lim) * k.dti, k.len, lim);
+  const double c =
+      dv.template over<kFace>(dv.template div<kFace>(left ? vel : -vel, Dv, lim) * k.dti, k.len, lim);
   fc.cfl = lim ? c : 0.0;
   if constexpr (SCH == P2_PDM) {
-    fc.E = dv.div(2.0, 1.0 - fc.cfl, lim);
+    fc.E = dv.template div<kBound>(2.0, 1.0 - fc.cfl, lim);
     fc.c1 = dv.den(fc.cfl + 1.e-10);
   } else {
     fc.E = 0.0;
@@ -196,13 +229,13 @@ __device__ __forceinline__ double reconstruct_bf(double cfl, double E, const Den
     // cfl >= 0, no operand is NaN and no two are zeros of opposite sign, so
     // v_min_f64 / v_max_f64 pick the operand the comparison form picks
     take = lim & (deltaf * deltafu > 0.0);
-    const double ratio = dv.div(deltafu, deltaf, take);
+    const double ratio = dv.template div<kNonzero>(deltafu, deltaf, take);
     double limiter;
     if constexpr (SCH == P2_PDM) {
       const double one6th = 1.0 / 6.0;
       const double x = one6th * (1.0 - 2.0 * cfl);
       limiter = (0.5 + x) + (0.5 - x) * ratio;
-      limiter = __builtin_fmin(__builtin_fmin(dv.over(2.0 * ratio, c1, take), limiter), E);
+      limiter = __builtin_fmin(__builtin_fmin(dv.template over<kRatio>(2.0 * ratio, c1, take), limiter), E);
     } else if constexpr (SCH == SUPERBEE) {
       (void)E;
       limiter = __builtin_fmax(__builtin_fmin(2.0 * ratio, 1.0), __builtin_fmin(ratio, 2.0));
@@ -357,9 +390,9 @@ template <int SCH, typename Div>
 __device__ __forceinline__ void wface_setup(WFace<true>& wf, double w, double dt, double Dlo,
                                             double Dhi, bool used, Div& dv) {
   wf.w = w;
-  wf.cfl = dv.div(__builtin_fabs(w) * dt, 0.5 * (Dlo + Dhi), used);
+  wf.cfl = dv.template div<kFace>(__builtin_fabs(w) * dt, 0.5 * (Dlo + Dhi), used);
   if constexpr (SCH == P2_PDM) {
-    wf.E = dv.div(2.0, 1.0 - wf.cfl * 1.0, used);
+    wf.E = dv.template div<kBound>(2.0, 1.0 - wf.cfl * 1.0, used);
     wf.c1 = dv.den(wf.cfl * 1.0 + 1.e-10);
   } else {
     wf.E = 0.0;

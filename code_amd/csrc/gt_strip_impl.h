@@ -73,10 +73,10 @@ __device__ __forceinline__ double rcp_nr(double x) {
 // rounding of 2^-1075.
 // A zero numerator gives +0 where the full sequence keeps its sign.
 // Cost and reach (400 x 400 x 40, two tracers, P2-PDM): 380 us where nothing
-// fires (375 with the remainder's class as the only test, 470 with full
-// divisions alone); tails of a tracer that fade out below 1e-292 fire it: a
-// patch in an empty basin after 30 / 300 steps 400 / 432 us (441 / 450), a
-// field that lies there as a whole 462 (469).
+// fires (375 with the remainder's class as the only test, 455 with full
+// divisions alone); tails of a tracer that fade out below 1e-292 fire it
+// (look_ahead has their figures), a field that lies there as a whole takes 441
+// (469 with full divisions alone).
 struct Den {
   double b, y;
 };
@@ -88,6 +88,7 @@ struct Den {
 // NaN for c = 1, which the min takes for the infinity it stands for.
 enum Quot { kAny, kNonzero, kFace, kRatio, kBound };
 struct DivFull {
+  static constexpr bool kTests = false;
   __device__ __forceinline__ Den den(double b) const { return {b, 0.0}; }
   template <Quot Q = kAny>
   __device__ __forceinline__ double over(double a, const Den& d, bool) const {
@@ -103,7 +104,13 @@ struct DivFull {
 struct DivNewton {
   uint64_t bad = 0;    // the lanes it fired on, up to the last pin()
   bool fired = false;  // and since
-  static constexpr uint32_t kLow = (1023 - 969) << 21;  // 2^-969's bits past the sign
+  static constexpr bool kTests = true;
+  // below 2^-969 and not zero: by the bits past the sign, less one, which
+  // makes a zero the largest
+  static __device__ __forceinline__ bool tiny(double a) {
+    const uint64_t m = (__builtin_bit_cast(uint64_t, a) << 1) - 1;
+    return (uint32_t)(m >> 32) < (1023 - 969) << 21;
+  }
   __device__ __forceinline__ Den den(double b) const {
     double y = __builtin_amdgcn_rcp(b);
     y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
@@ -120,9 +127,7 @@ struct DivNewton {
     if constexpr (Q == kNonzero) {
       fired |= used & ((__builtin_fabs(a) < 0x1p-969) | __builtin_amdgcn_class(q, kNanInfDenorm));
     } else if constexpr (Q == kAny) {
-      // the bits past the sign, less one: a zero comes out largest
-      const uint64_t m = (__builtin_bit_cast(uint64_t, a) << 1) - 1;
-      fired |= used & (((uint32_t)(m >> 32) < kLow) | __builtin_amdgcn_class(q, kNanInfDenorm));
+      fired |= used & (tiny(a) | __builtin_amdgcn_class(q, kNanInfDenorm));
     } else if constexpr (Q != kBound) {
       fired |= used & __builtin_amdgcn_class(r, kNanInfDenorm);
     }
@@ -131,6 +136,11 @@ struct DivNewton {
   template <Quot Q = kAny>
   __device__ __forceinline__ double div(double a, double b, bool used) {
     return over<Q>(a, den(b), used);
+  }
+  // fires for a tracer value that a quotient will fire for, from its high word
+  // (values below 2^-1042 pass)
+  __device__ __forceinline__ void look(uint32_t hi, bool used) {
+    fired |= used & ((hi << 1) - 1 < (1023 - 969) << 21);
   }
   // ends a section of the row: the tests of the section's quotients stay in
   // it (left to the compiler they gather at the row's end and keep every
@@ -561,6 +571,31 @@ enum { MOM_NONE = 0, MOM_U = 1, MOM_V = 2 };
 // instead of five that read them (256 x 256 x 30, one FP64 tracer: 83 us
 // against 117; 320 x 256 x 30 x 18 FP32: 695 against 773).
 
+// Five rows spread over a strip's nsteps are looked at before the march, so
+// that a strip in a tail (which runs over several rows) takes the full
+// divisions at once and not after a part of the short march: 400 x 400 x 40,
+// two tracers, 40 patches in an empty basin after 60 steps 441 us against 481
+// (449 with full divisions alone); nothing tiny, 383 against 380.  Three rows
+// find fewer (478).  4-row strips lose little and are bound by latency: not
+// there.  load(s, g, fl): the high word of tracer g in the row of step s, fl
+// the cell's masks.
+template <int G, typename Div, typename Load>
+__device__ __forceinline__ void look_ahead(Div& dv, int nsteps, Load load) {
+  constexpr int N = 5;
+  const int stride = nsteps / N;
+  uint32_t f[N][G];
+  int fl[N];
+#pragma unroll
+  for (int q = 0; q < N; q++)
+#pragma unroll
+    for (int g = 0; g < G; g++) f[q][g] = load(stride / 2 + q * stride, g, fl[q]);
+#pragma unroll
+  for (int q = 0; q < N; q++)
+#pragma unroll
+    for (int g = 0; g < G; g++) dv.look(f[q][g], (fl[q] & MB_WCOL) != 0);
+  dv.pin();
+}
+
 // ---- kernel 1: u/2 then v/2 at level L ------------------------------------------------
 // Div: the divisions of the exact flavour; dv tells whether one left their
 // range
@@ -810,6 +845,16 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
   constexpr std::false_type off{};
   Row r;
   if constexpr (kRowAhead<TF>) load_row(y0 - 2, r);
+  if constexpr (Div::kTests && !MOM) {
+    if (nsteps > 8) {
+      look_ahead<G>(dv, nsteps, [&](int s, int g, int& fl) {
+        const uint32_t c = cell(y0 - 2 + s);
+        fl = flags[c] & cb.xin;
+        return ldo((const uint32_t*)fin_g[g], c * 8u + 4u);
+      });
+      if (dv.stop()) return;
+    }
+  }
   step(Slot<0>{}, off, off, r, 0);
   if (dv.stop()) return;
   step(Slot<1>{}, off, off, r, 1);
@@ -1200,6 +1245,16 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
   constexpr std::false_type off{};
   Row r;
   if constexpr (kRowAhead<TF>) load_row(y0 - 2, r);
+  if constexpr (Div::kTests && !MOM) {
+    if (nsteps > 8) {
+      look_ahead<G>(dv, nsteps, [&](int s, int g, int& fl) {
+        const uint32_t c = cell(y0 - 2 + s);
+        fl = flags[c] & cb.xin;
+        return ldo((const uint32_t*)f2_g[g], c * 8u + (lvo[2] + 4u));
+      });
+      if (dv.stop()) return;
+    }
+  }
   step(Slot<0>{}, off, off, r, 0);
   if (dv.stop()) return;
   step(Slot<1>{}, off, off, r, 1);

@@ -88,3 +88,28 @@ def test_courant_number_one(device, scheme, sign):
     f = inputs.uniform((2,) + sh, 91, -1.0, 3.0)
     got, want = both(device, dom, F, f, scheme)
     assert np.array_equal(got, want, equal_nan=True), int((got != want).sum())
+
+
+@pytest.mark.parametrize("scheme", SCHEMES)
+@pytest.mark.parametrize("rows", [8, 16, 32])
+def test_tails_through_part_of_the_strips(device, scheme, rows):
+    """a tracer that falls off by 10**-3 per cell around two patches: strips
+    before, in and past the tail, and tiny values on land"""
+    dom = random_domain(190, 120, 4, 9, "islands")
+    F = random_fields(dom, 419, cmax=0.3, plateaus=False)
+    j, i = np.mgrid[:dom.NY, :dom.NX]
+    f = np.zeros((2,) + dom.shape3)
+    for t, (cj, ci) in enumerate(((9, 150), (61, 20))):
+        d = np.abs(j - cj) + np.abs(i - ci)
+        f[t, 1:] = inputs.uniform((dom.kmax,) + d.shape, 95 + t, 1.0, 9.0) * 10.0 ** (-3.0 * d)
+    orc = po.Oracle.from_domain(dom)
+    ctx = gt.Context.from_domain(dom)
+    ctx.set_tuning(fused=1, tile=gt.tile_for_rows(rows), group=2)
+    out = torch.empty(f.shape, dtype=torch.float64, device=device)
+    gt.adv3d_batch([dict(ctx=ctx, f_in=to_dev(f, device), f_out=out,
+                         **{n: to_dev(F[n], device) for n in VEL})], 2, F["dt"], scheme, scheme)
+    got = to_host(out)
+    for t in range(2):
+        orc.do_advection_3d(F["dt"], f[t], *(F[n] for n in VEL), F["ho"], gt.HALFSPLIT, scheme,
+                            scheme, -1.0, gt.H_TAG)
+        assert np.array_equal(got[t], f[t]), (t, int((got[t] != f[t]).sum()))

@@ -168,17 +168,17 @@ struct CellOp<false> {
   float am1 = 0.0f, b = 0.0f;
   // dtc = dt*splitfac*dlen*ard1 (dt for w)
   __device__ static CellOp make(double Dio, double Dn, double dtc) {
-    const CellK k = cell_factors(true, Dio, Dn, dtc);
+    const CellK k = cell_factors(Dio, Dn, dtc);
     CellOp c;
     c.am1 = k.am1;
     c.b = k.b;
     return c;
   }
   __device__ float h_step(float fo, float Fc, float Fm, double, double, double) const {
-    return cell_update_fast(CellK{am1, b}, fo, Fc, Fm);
+    return cell_update_fast(true, CellK{am1, b}, fo, Fc, Fm);
   }
   __device__ float w_step(float fo, float wk, float wprev, double) const {
-    return cell_update_fast(CellK{am1, b}, fo, wk, wprev);
+    return cell_update_fast(true, CellK{am1, b}, fo, wk, wprev);
   }
   __device__ float diag(float l) const { return __builtin_fmaf(l, am1, l); }
   __device__ float mu(float l, double, double) const { return -b * l; }

@@ -10,7 +10,9 @@
 
 #include <cmath>
 #include <cstdarg>
+#include <cstdint>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -1063,7 +1065,13 @@ extern "C" int gt_uv_advect_3d(gt_ctx* c, double dt, const double* uu, const dou
     if (!p) return set_err(GT_EARG, "gt_uv_advect_3d: NULL argument");
   if (hscheme == GT_J7) return set_err(GT_ENOTIMPL, "uv_advect_3d: J7 is not in this build");
   if (hscheme == GT_NOADV && vscheme == GT_NOADV) return GT_OK;
-  if (split == GT_HALFSPLIT && c->fused && c->adv_ver_iterations <= 1 && c->kmax > 1 &&
+  // The strip kernels read the caller's fields while neighbouring strips write
+  // the results, so results that lie in an input take the way through copies
+  bool apart = true;
+  for (int q = 0; q < 7; q++)
+    for (int r = 7; r < 9; r++)
+      apart &= (size_t)std::llabs((intptr_t)ps[q] - (intptr_t)ps[r]) >= sizeof(double) * c->N3;
+  if (split == GT_HALFSPLIT && c->fused && c->adv_ver_iterations <= 1 && c->kmax > 1 && apart &&
       gt::fused_supported(hscheme, vscheme) && strip_fits(c)) {
     const size_t ws = strip_ws_bytes(c, sizeof(double), 1, true);
     TRY(ensure_ws(c, ws + sizeof(double) * (size_t)c->d.NX * (c->kmax + 1)));

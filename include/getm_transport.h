@@ -196,8 +196,11 @@ int gt_ww_momentum_3d(gt_ctx *ctx, double dt, const double *uu,
  * (GT_ENOTIMPL) and without the numerical analyses: u = uu/hun on the U
  * control volumes, with the transports, ww and the layer heights averaged
  * onto them, advected by do_advection_3d (tag U_TAG, AH = 0), advection term
- * into uuEx; the same on the V volumes into vvEx.  The context keeps six
- * work fields (the reference's automatic arrays). */
+ * into uuEx; the same on the V volumes into vvEx.  HALFSPLIT with one scheme
+ * forms the averages in the strip kernels; the other calls, and those whose
+ * uuEx or vvEx overlaps an input, in six work fields that the context keeps
+ * (the reference's automatic arrays).  uuEx must not overlap hun, nor vvEx
+ * hvn. */
 int gt_uv_advect_3d(gt_ctx *ctx, double dt, const double *uu, const double *vv,
                     const double *ww, const double *ho, const double *hn,
                     const double *hun, const double *hvn, int split,

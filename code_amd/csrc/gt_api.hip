@@ -478,8 +478,15 @@ static size_t strip_ws_bytes(const gt_ctx* c, size_t tf_bytes, int ntracers, boo
 static long budget_strip_levels(const gt_ctx* c) {
   return (long)((c->d.NX + gt::kStripOut - 1) / gt::kStripOut) * ((c->d.NY + 3) / 4) * c->kmax;
 }
-static size_t budget_ws_bytes(const gt_ctx* c, int ntracers) {
-  return sizeof(double) * 2 * (size_t)(ntracers + 1) * (size_t)budget_strip_levels(c);
+// where a batch's partials start in its work fields (pairs, read 16 bytes at a
+// time), and the work fields with them
+static size_t budget_offset(const gt_ctx* c, size_t tf_bytes, int ntracers) {
+  return (strip_ws_bytes(c, tf_bytes, ntracers, false) + 15) / 16 * 16;
+}
+static size_t batch_ws_bytes(const gt_ctx* c, size_t tf_bytes, int ntracers, bool budget) {
+  if (!budget) return strip_ws_bytes(c, tf_bytes, ntracers, false);
+  return budget_offset(c, tf_bytes, ntracers) +
+         sizeof(double) * 2 * (size_t)(ntracers + 1) * (size_t)budget_strip_levels(c);
 }
 
 // the HALFSPLIT and FULLSPLIT sub-steps of ns slices from level k0 in two
@@ -1383,10 +1390,8 @@ extern "C" int gt_reserve(gt_ctx* c, int ntracers_f32, int ntracers_f64) {
   // the batched step's work fields with room for the budgets formed in it
   size_t ws = strip_ws_bytes(c, sizeof(double), 1, true) +
               sizeof(double) * (size_t)c->d.NX * (c->kmax + 1);  // (and uv_advect_3d's row)
-  const size_t w32 = strip_ws_bytes(c, sizeof(float), ntracers_f32, false) +
-                     (ntracers_f32 > 0 ? budget_ws_bytes(c, ntracers_f32) : 0);
-  const size_t w64 = strip_ws_bytes(c, sizeof(double), ntracers_f64, false) +
-                     (ntracers_f64 > 0 ? budget_ws_bytes(c, ntracers_f64) : 0);
+  const size_t w32 = batch_ws_bytes(c, sizeof(float), ntracers_f32, ntracers_f32 > 0);
+  const size_t w64 = batch_ws_bytes(c, sizeof(double), ntracers_f64, ntracers_f64 > 0);
   if (w32 > ws) ws = w32;
   if (w64 > ws) ws = w64;
   TRY(ensure_ws(c, ws));
@@ -1523,8 +1528,7 @@ static int batch_impl(int ndom, const gt_batch_domain* doms, int ntracers, doubl
   }
   for (int i = 0; i < ndom; i++) {
     gt_ctx* c = doms[i].ctx;
-    TRY(ensure_ws(c, strip_ws_bytes(c, sizeof(TF), ntracers, false) +
-                         (doms[i].budget ? budget_ws_bytes(c, ntracers) : 0)));
+    TRY(ensure_ws(c, batch_ws_bytes(c, sizeof(TF), ntracers, doms[i].budget != nullptr)));
   }
   for (int b = 0; b < ndom; b += gt::kMaxFusedDomains) {
     gt::FusedArgs<TF> A{};
@@ -1537,7 +1541,7 @@ static int batch_impl(int ndom, const gt_batch_domain* doms, int ntracers, doubl
                       nullptr);
       // the budget partials follow the work fields
       if (bd.budget)
-        A.doms[i].bpart = (double*)((char*)c->ws + strip_ws_bytes(c, sizeof(TF), ntracers, false));
+        A.doms[i].bpart = (double*)((char*)c->ws + budget_offset(c, sizeof(TF), ntracers));
     }
     A.ndom = nd;
     A.ntracers = ntracers;

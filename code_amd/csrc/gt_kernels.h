@@ -143,7 +143,8 @@ hipError_t launch_budget_batch(hipStream_t st, Dims d, const int32_t* az, int nt
                                double area, double* out);
 // the final pass alone, for up to 8 domains in one launch: for domain i,
 // out[q] = area * (sum of the npairs (hi, lo) pairs at partial + 2*q*npairs),
-// q < nout, in k_budget_batch_final's order
+// q < nout, in double-double (1024 threads with four sums each, then a tree);
+// partial must lie on 16 bytes
 struct BudgetPairs {
   const double* partial;
   double* out;

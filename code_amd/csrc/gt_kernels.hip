@@ -1257,7 +1257,10 @@ hipError_t launch_budget_batch(hipStream_t st, Dims d, const int32_t* az, int nt
 
 hipError_t launch_budget_pairs_final(hipStream_t st, const BudgetPairsSet& S) {
   long nblocks = 0;
-  for (int i = 0; i < S.n; i++) nblocks += S.d[i].nout;
+  for (int i = 0; i < S.n; i++) {
+    if ((uintptr_t)S.d[i].partial % sizeof(double2)) return hipErrorInvalidValue;
+    nblocks += S.d[i].nout;
+  }
   if (nblocks == 0) return hipSuccess;
   hipLaunchKernelGGL(k_budget_pairs_final, dim3((unsigned)nblocks), dim3(kPairThreads), 0, st,
                      S);

@@ -503,15 +503,16 @@ static int strips_2d(gt_ctx* c, const GridMasks* g, int k0, int ns, double dt, d
                      const double* Do, int split, int scheme, double AH, double* Dires,
                      double* advres) {
   const bool half = split == GT_HALFSPLIT;
-  const long NXY = c->d.NXY, o = NXY * k0;
-  TRY(ensure_ws(c, strip_ws_bytes(c, sizeof(double), 1, advres != nullptr)));
+  const long NXY = c->d.NXY, o = NXY * k0, n = NXY * ns;
+  // work fields of these slices alone: a depth-mean call needs no 3-D field
+  TRY(ensure_ws(c, sizeof(double) * n * (advres ? 3 : 2)));
   gt::FusedArgs<double> A{};
   gt::FusedDomain<double>& D = A.doms[0];
   // the kernel's levels are 1..ns: the bases lie one slice below
   const long b = o - NXY;
   fill_domain<double>(c, g, &D, f + b, nullptr, 0, 1, U + b, V + b, nullptr, DU + b, DV + b,
                       Do + b, nullptr, advres);
-  double *f2 = D.f2, *d2 = D.d2, *a2 = D.a2;
+  double *d2 = (double*)c->ws, *f2 = d2 + n, *a2 = advres ? f2 + n : nullptr;
   D.f2 = f2 - NXY;
   D.d2 = d2 - NXY;
   if (a2) D.a2 = a2 - NXY;
@@ -533,7 +534,7 @@ static int strips_2d(gt_ctx* c, const GridMasks* g, int k0, int ns, double dt, d
     LCHK(gt::launch_half_u(c->st, c->d, ns, f2, d2, a2, f + o, di, ad, U + o, DU + o, g->flags, dt,
                            c->dx, c->dy, c->ard1, scheme, AH));
   else
-    LCHK(gt::launch_copy3(c->st, NXY * ns, f + o, f2, di, d2, ad, a2));
+    LCHK(gt::launch_copy3(c->st, n, f + o, f2, di, d2, ad, a2));
   return GT_OK;
 }
 

@@ -15,6 +15,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "../../include/getm_transport.h"
@@ -1371,10 +1372,10 @@ extern "C" int gt_exchange_tiles(int px, int py, const int* ni, const int* nj, i
 // ---- batched multi-tracer step (extension) ----------------------------------
 extern "C" int gt_set_tuning(gt_ctx* c, int fused, int tile, int group) {
   if (!c) return set_err(GT_EARG, "gt_set_tuning: NULL context");
-  if (tile < 0 || tile > 11)
-    return set_err(GT_EARG, "gt_set_tuning: tile must be 0..11 (rows per strip, see the header)");
-  if (group != 1 && group != 2 && group != 3 && group != 6 && group != 9)
-    return set_err(GT_EARG, "gt_set_tuning: group must be 1, 2, 3, 6 or 9");
+  if (tile < -1 || tile > 12)
+    return set_err(GT_EARG, "gt_set_tuning: tile must be -1..12 (rows per strip, see the header)");
+  if (group != 0 && group != 1 && group != 2 && group != 3 && group != 6 && group != 9)
+    return set_err(GT_EARG, "gt_set_tuning: group must be 0, 1, 2, 3, 6 or 9");
   c->fused = fused != 0;
   c->tile = tile;
   c->group = group;
@@ -1590,70 +1591,103 @@ extern "C" int gt_adv3d_batch_f64(int ndom, const gt_batch_domain* doms, int ntr
 // ---- autotuner (extension) ------------------------------------------------------
 // Times the batched step for every rows-per-strip x tracers-per-wavefront pair
 // (reps launches each, after one warm-up) with HIP events on the stream and
-// keeps the fastest on every context of the batch.  Outputs are written to
-// f_out (f_in is not modified), so the sweep can run on live buffers.
+// keeps the fastest on every context of the batch; after an error each context
+// has its own choice back.  Outputs are written to f_out (f_in is not
+// modified), so the sweep can run on live buffers.
+namespace {
+struct SweepState {
+  int ndom;
+  const gt_batch_domain* doms;
+  std::vector<std::pair<int, int>> had;  // the contexts' tile and group
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  SweepState(int n, const gt_batch_domain* d) : ndom(n), doms(d) {
+    for (int i = 0; i < n; i++) had.emplace_back(d[i].ctx->tile, d[i].ctx->group);
+  }
+  void set(int tile, int group) const {
+    for (int i = 0; i < ndom; i++) {
+      doms[i].ctx->tile = tile;
+      doms[i].ctx->group = group;
+    }
+  }
+  void keep(int tile, int group) {
+    set(tile, group);
+    had.clear();
+  }
+  ~SweepState() {
+    for (size_t i = 0; i < had.size(); i++) {
+      doms[i].ctx->tile = had[i].first;
+      doms[i].ctx->group = had[i].second;
+    }
+    if (e0) (void)hipEventDestroy(e0);
+    if (e1) (void)hipEventDestroy(e1);
+  }
+};
+}  // namespace
+
+// whether a launch left to itself takes the 4-row strips (which pay where they
+// fit the chip at once, and are not worth a measurement elsewhere)
+static bool takes_short_strips(int ndom, const gt_batch_domain* doms, int ntracers, int group,
+                               bool f32) {
+  gt::FusedArgs<float> A{};
+  gt::FusedArgs<double> B{};
+  A.ndom = B.ndom = ndom < gt::kMaxFusedDomains ? ndom : gt::kMaxFusedDomains;
+  A.ntracers = B.ntracers = ntracers;
+  for (int i = 0; i < A.ndom; i++) A.doms[i].d = B.doms[i].d = doms[i].ctx->d;
+  gt::strip_auto_rows(A, group);
+  gt::strip_auto_rows(B, group);
+  return (f32 ? A.rows[0] : B.rows[0]) == 4;
+}
+
 extern "C" int gt_autotune_batch(int ndom, const gt_batch_domain* doms, int ntracers, double dt,
                                  int hscheme, int vscheme, double AH, int tag, int f32, int reps,
                                  void* stream, int* best_tile, int* best_group, float* best_ms,
                                  float* table) {
-  if (ndom < 1 || !doms || !doms[0].ctx || reps < 1)
+  if (ndom < 1 || !doms || ntracers < 1 || reps < 1)
     return set_err(GT_EARG, "gt_autotune_batch: bad argument");
+  for (int i = 0; i < ndom; i++)
+    if (!doms[i].ctx) return set_err(GT_EARG, "gt_autotune_batch: domain %d has no context", i);
   hipStream_t st = stream ? (hipStream_t)stream : doms[0].ctx->st;
-  // strip heights of the two kernels: 9 pairs {16, 32, 8} x {16, 32, 8}
-  const int tiles[9] = {3, 4, 5, 6, 7, 8, 9, 10, 11};
+  // strip heights of the two kernels: 9 pairs {16, 32, 8} x {16, 32, 8}, then
+  // 4 rows for both (not in the table)
+  const int tiles[10] = {3, 4, 5, 6, 7, 8, 9, 10, 11, 12};
   const int groups[4] = {1, 3, 6, 9};
   const int groups64[2] = {1, 2};
-  hipEvent_t e0, e1;
-  HIPCHK(hipEventCreate(&e0));
-  HIPCHK(hipEventCreate(&e1));
+  const int ng = f32 ? 4 : 2;
+  SweepState S(ndom, doms);
+  HIPCHK(hipEventCreate(&S.e0));
+  HIPCHK(hipEventCreate(&S.e1));
   float best = 1e30f;
   int bt = 0, bg = 3;
   // two passes over the candidates, each candidate's time the lower of its
   // two: a transient slowdown of the device then moves no choice
-  float tmin_ms[36];
-  for (int q = 0; q < 36; q++) tmin_ms[q] = 1e30f;
-  for (int pass = 0; pass < 2; pass++) {
-  int n = 0;
-  for (int ti = 0; ti < 9; ti++)
-    for (int gi = 0; gi < (f32 ? 4 : 2); gi++) {
-      const int grp = f32 ? groups[gi] : groups64[gi];
-      for (int i = 0; i < ndom; i++) {
-        doms[i].ctx->tile = tiles[ti];
-        doms[i].ctx->group = grp;
-      }
+  float tmin_ms[40];
+  for (int q = 0; q < 40; q++) tmin_ms[q] = 1e30f;
+  for (int pass = 0; pass < 2; pass++)
+    for (int n = 0; n < 10 * ng; n++) {
+      const int tile = tiles[n / ng], grp = f32 ? groups[n % ng] : groups64[n % ng];
+      if (tile == 12 && !takes_short_strips(ndom, doms, ntracers, grp, f32)) continue;
+      S.set(tile, grp);
       auto run = [&]() -> int {
         return f32 ? gt_adv3d_batch_f32(ndom, doms, ntracers, dt, hscheme, vscheme, AH, tag, st)
                    : gt_adv3d_batch_f64(ndom, doms, ntracers, dt, hscheme, vscheme, AH, tag, st);
       };
-      int rc = run();
-      if (rc != GT_OK) {
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
-        return rc;
-      }
-      HIPCHK(hipEventRecord(e0, st));
+      TRY(run());
+      HIPCHK(hipEventRecord(S.e0, st));
       for (int r = 0; r < reps; r++) TRY(run());
-      HIPCHK(hipEventRecord(e1, st));
-      HIPCHK(hipEventSynchronize(e1));
+      HIPCHK(hipEventRecord(S.e1, st));
+      HIPCHK(hipEventSynchronize(S.e1));
       float ms = 0.f;
-      HIPCHK(hipEventElapsedTime(&ms, e0, e1));
+      HIPCHK(hipEventElapsedTime(&ms, S.e0, S.e1));
       ms /= reps;
       ms = tmin_ms[n] = ms < tmin_ms[n] ? ms : tmin_ms[n];
-      if (table) table[n] = ms;
-      n++;
+      if (table && tile != 12) table[n] = ms;
       if (pass == 1 && ms < best) {
         best = ms;
-        bt = tiles[ti];
+        bt = tile;
         bg = grp;
       }
     }
-  }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  for (int i = 0; i < ndom; i++) {
-    doms[i].ctx->tile = bt;
-    doms[i].ctx->group = bg;
-  }
+  S.keep(bt, bg);
   if (best_tile) *best_tile = bt;
   if (best_group) *best_group = bg;
   if (best_ms) *best_ms = best;

@@ -67,7 +67,8 @@ struct FusedArgs {
 
 // rows per strip for a tuning index: 0 -> 16, 1 -> 32, 2 -> 8 for both
 // kernels; 3..11 -> the first kernel {16, 32, 8}[(t-3)%3], the second
-// {16, 32, 8}[(t-3)/3] (multiples of 4: the row march is unrolled four times)
+// {16, 32, 8}[(t-3)/3]; 12 -> 4 for both (multiples of 4: the row march is
+// unrolled four times)
 void strip_rows(int tile, int rows[2]);
 // the choice where the caller made none (gt_set_tuning): tracers per
 // wavefront, and rows per strip (4, 8, 16 or 32) given them; the caller has

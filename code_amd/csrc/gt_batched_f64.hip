@@ -6,7 +6,9 @@ namespace gt {
 
 void strip_rows(int tile, int rows[2]) {
   static const int r[3] = {16, 32, 8};
-  if (tile >= 3 && tile < 12) {
+  if (tile == 12) {
+    rows[0] = rows[1] = 4;
+  } else if (tile >= 3 && tile < 12) {
     rows[0] = r[(tile - 3) % 3];
     rows[1] = r[(tile - 3) / 3];
   } else {

@@ -723,6 +723,9 @@ class Context:
                                              self._f3(S_bar, "S_bar", True), dtr0, dsr0))
 
     def set_tuning(self, fused=1, tile=0, group=3):
+        """gt_set_tuning: kernel choice, strip heights (an index for strip_rows;
+        -1: the library's choice) and tracers per wavefront (0: the library's
+        choice).  The defaults pin 16 rows and groups of 3."""
         check(self.lib.gt_set_tuning(self.h, int(fused), int(tile), int(group)))
 
     def set_adjoint_mode(self, keep_states=-1):
@@ -788,12 +791,14 @@ def _batch_array(domains, ntracers):
 
 # strip heights of the HALFSPLIT strip kernels; a tuning index t < 3 gives
 # ROWS[t] rows to both kernels, 3 <= t < 12 gives ROWS[(t-3)%3] to the first
-# (u/2 v/2) and ROWS[(t-3)//3] to the second (w v/2 u/2)
+# (u/2 v/2) and ROWS[(t-3)//3] to the second (w v/2 u/2), t = 12 gives 4 to both
 ROWS = (16, 32, 8)
 
 
 def strip_rows(tile):
     """(rows of the first kernel, rows of the second) for a tuning index"""
+    if tile == 12:
+        return 4, 4
     if 3 <= tile < 12:
         return ROWS[(tile - 3) % 3], ROWS[(tile - 3) // 3]
     r = ROWS[tile if 0 <= tile < 3 else 0]
@@ -801,17 +806,21 @@ def strip_rows(tile):
 
 
 def tile_for_rows(rows_uv, rows_wvu=None):
-    """the tuning index of a strip-height pair (8, 16 or 32 rows each)"""
+    """the tuning index of a strip-height pair (8, 16 or 32 rows each, or 4 for
+    both)"""
     rows_wvu = rows_uv if rows_wvu is None else rows_wvu
+    if rows_uv == rows_wvu == 4:
+        return 12
     if rows_uv not in ROWS or rows_wvu not in ROWS:
-        raise ValueError(f"rows per strip must be one of {sorted(ROWS)}")
+        raise ValueError(f"rows per strip must be one of {sorted(ROWS)}, or 4 for both")
     return 3 + ROWS.index(rows_uv) + 3 * ROWS.index(rows_wvu)
 
 
 def autotune_batch(domains, ntracers, dt, hscheme, vscheme, AH=-1.0, tag=H_TAG, reps=3,
                    stream=None):
     """gt_autotune_batch: returns (tile, group, best_ms, {(tile, group): ms}); tile
-    is a strip-height index (strip_rows), group the tracers per wavefront"""
+    is a strip-height index (strip_rows), group the tracers per wavefront; the
+    4-row strips it may choose on a small grid are not in the table"""
     import torch
     lib = load_library()
     arr = _batch_array(domains, ntracers)

@@ -436,12 +436,13 @@ int gt_adv3d_batch_f64(int ndom, const gt_batch_domain *doms, int ntracers,
  * per-sub-step kernels (0; gt_adv3d_batch_f32 then runs the FP32 sub-steps
  * one kernel each, bit-identical to the strip kernels, and accepts
  * hscheme != vscheme; gt_adv3d_batch_f64 always runs the strip kernels);
- * rows per strip (default, without this call: 4 to 32 by the number of
- * strip-levels of each launch): tile 0, 1, 2 give 16, 32, 8 rows
+ * rows per strip (tile -1, the default without this call: 4 to 32 by the
+ * number of strip-levels of each launch): tile 0, 1, 2 give 16, 32, 8 rows
  * to both kernels, tile 3..11 gives {16, 32, 8}[(tile-3)%3] rows to the first
- * (u/2 v/2) and {16, 32, 8}[(tile-3)/3] to the second (w v/2 u/2); tracers
- * per wavefront (group: FP32 1, 3, 6 or 9; FP64 1, or 2 for any other value
- * when there are two or more tracers) */
+ * (u/2 v/2) and {16, 32, 8}[(tile-3)/3] to the second (w v/2 u/2), tile 12
+ * gives 4 rows to both; tracers per wavefront (group 0, the default: by the
+ * number of tracers and of strip-levels; else FP32 1, 3, 6 or 9, FP64 1, or 2
+ * for any other value when there are two or more tracers) */
 int gt_set_tuning(gt_ctx *ctx, int fused, int tile, int group);
 /* reverse mode (gt_adv3d_adjoint*): keep_states 1 keeps the four sub-step
  * states of every step of a checkpoint segment while the segment is
@@ -465,11 +466,14 @@ int gt_set_adjoint_mode(gt_ctx *ctx, int keep_states);
  * arrays (do_advection_3d fi/hi/adv, SMcW dR/dZ/P). */
 int gt_reserve(gt_ctx *ctx, int ntracers_f32, int ntracers_f64);
 /* autotuner: times gt_adv3d_batch_f32 (f32=1) or _f64 over the nine strip
- * height pairs (tile 3..11) x tracers per wavefront {1, 3, 6, 9} (FP64:
- * {1, 2}), reps timed launches each, in two passes over the candidates,
- * and keeps the fastest on every context.  table (optional, 36 floats)
- * receives each pair's ms (the lower of its two passes' means) in sweep
- * order (tile outer).  f_out is overwritten, f_in is not touched. */
+ * height pairs (tile 3..11), and 4 rows (tile 12) where the default would
+ * take them, x tracers per wavefront {1, 3, 6, 9} (FP64: {1, 2}), reps timed
+ * launches each, in two passes over the candidates, and keeps the fastest on
+ * every context (gt_set_tuning with tile -1 and group 0 goes back to the
+ * default); after an error each context has the choice it had.  table
+ * (optional, 36 floats) receives the ms of each of the nine pairs (the lower
+ * of its two passes' means) in sweep order (tile outer).  f_out is
+ * overwritten, f_in is not touched. */
 int gt_autotune_batch(int ndom, const gt_batch_domain *doms, int ntracers,
                       double dt, int hscheme, int vscheme, double AH, int tag,
                       int f32, int reps, void *hip_stream, int *best_tile,

@@ -1415,6 +1415,12 @@ extern "C" int gt_set_adjoint_mode(gt_ctx* c, int keep_states) {
   if (!c) return set_err(GT_EARG, "gt_set_adjoint_mode: NULL context");
   if (keep_states < -1 || keep_states > 1)
     return set_err(GT_EARG, "gt_set_adjoint_mode: keep_states must be -1, 0 or 1");
+  if (c->adj_keep != keep_states && c->w32) {
+    HIPCHK(hipDeviceSynchronize());  // the fields may still be in use
+    HIPCHK(hipFree(c->w32));
+    c->w32 = nullptr;
+    c->w32_bytes = 0;
+  }
   c->adj_keep = keep_states;
   return GT_OK;
 }
@@ -1765,16 +1771,26 @@ static int adjoint_impl(const char* name, gt_ctx* c, int ntr, int nsteps, int ck
   const long N3 = c->N3;
   const size_t set = (size_t)ntr * N3;
   // With the choice left to the library and the states of the whole window in
-  // an eighth of the free memory, the window is one segment: nothing is
-  // recomputed (the checkpoint spacing changes no result): 256 x 256 x 30 x
-  // 48 steps, checkpoint every 8, 3.1 ms less per call (of 14.5), 4.1 GB.
+  // an eighth of the free memory, or in what the context holds already, the
+  // window is one segment whose states are kept: nothing is recomputed (the
+  // checkpoint spacing changes no result): 256 x 256 x 30 x 48 steps,
+  // checkpoint every 8, 3.1 ms less per call (of 14.5), 4.1 GB.
+  bool keep = c->adj_keep == 1;
+  size_t avail = 0;
+  if (c->adj_keep < 0) {
+    size_t fr = 0, tot = 0;
+    if (hipMemGetInfo(&fr, &tot) == hipSuccess) avail = fr + c->w32_bytes;
+    else (void)hipGetLastError();
+  }
+  auto fits = [&](size_t bytes, int share) {
+    return bytes <= c->w32_bytes || bytes <= avail / share;
+  };
   if (c->adj_keep < 0 && ckpt_every < nsteps) {
     const size_t all = sizeof(double) * 5 * (size_t)N3 * (in.per_step ? nsteps : 1) +
                        sizeof(TF) * (5 * (size_t)nsteps + 2) * set;
-    size_t fr = 0, tot = 0;
-    if (all <= c->w32_bytes ||
-        (hipMemGetInfo(&fr, &tot) == hipSuccess && all <= (fr + c->w32_bytes) / 8)) {
-      if (ensure_w32(c, all) == GT_OK) ckpt_every = nsteps;
+    if (fits(all, 8)) {
+      keep = ensure_w32(c, all) == GT_OK;
+      if (keep) ckpt_every = nsteps;
       else (void)hipGetLastError();
     }
   }
@@ -1786,17 +1802,13 @@ static int adjoint_impl(const char* name, gt_ctx* c, int ntr, int nsteps, int ck
   // lam[2], the checkpoints and the seg-1 states inside a segment.  Keeping
   // the states lets the reverse steps skip the four sub-steps that would
   // recover them; it is taken when asked for, or (default) when it needs at
-  // most half of the free device memory.
+  // most half of the free device memory or the context holds what it needs.
   const size_t rest = 2 + (size_t)nck + (size_t)(seg - 1);
   auto bytes_for = [&](bool k) -> size_t {
     const size_t hs = k && in.per_step ? (size_t)seg : 1;
     return sizeof(double) * 5 * (size_t)N3 * hs + sizeof(TF) * ((k ? 4 * (size_t)seg : 4) + rest) * set;
   };
-  bool keep = c->adj_keep == 1;
-  if (c->adj_keep < 0) {
-    size_t fr = 0, tot = 0;
-    if (hipMemGetInfo(&fr, &tot) == hipSuccess) keep = bytes_for(true) <= (fr + c->w32_bytes) / 2;
-  }
+  if (c->adj_keep < 0 && !keep) keep = fits(bytes_for(true), 2);
   int got = ensure_w32(c, bytes_for(keep));
   if (got != GT_OK && keep && c->adj_keep < 0) {
     // the free memory was there but not in one piece: recompute instead

@@ -452,8 +452,12 @@ int gt_set_tuning(gt_ctx *ctx, int fused, int tile, int group);
  * reverse step; -1 (default) keeps them when that needs at most half of the
  * free device memory, and treats the whole window as one segment
  * (ckpt_every = nsteps, nothing recomputed) when that needs at most an eighth
- * of it.  Results are the same bit for bit.  No counterpart in
- * the reference (its reverse mode is this build's extension). */
+ * of it; either also when the work memory the context holds is enough.  With
+ * 0 and 1 ckpt_every bounds the work memory as gt_adv3d_adjoint says.  A
+ * change of the mode gives the work memory back (it is allocated again on
+ * demand); otherwise the context holds it.  Results are the same bit for bit.
+ * No counterpart in the reference (its reverse mode is this build's
+ * extension). */
 int gt_set_adjoint_mode(gt_ctx *ctx, int keep_states);
 /* sizes the context's work fields for the transport step up front (the
  * HALFSPLIT step with advres, batched steps of up to ntracers_f32 FP32 or

@@ -370,9 +370,7 @@ __device__ __forceinline__ double cell_update_exact(bool upd, double Dio, const 
 // (CellK); the bracket is a small correction, so their few FP32 roundings
 // are far below the final rounding of fo + correction.
 // A cell that is not updated is selected, not given zero factors: a NaN or an
-// infinity times zero is NaN, which would walk through land a cell per sub-step
-// (the selects, with those of the missing w faces, take 3%: 18 tracers on eight
-// subdomains 2.45 -> 2.53 ms).
+// infinity times zero is NaN, which would walk through land a cell per sub-step.
 struct CellK {
   float am1, b;
 };
@@ -551,7 +549,10 @@ __device__ __forceinline__ void sto(T* base, uint32_t off, T v) {
 // kernel and the shared fields loaded where a row starts).  FP32 loads where
 // the row starts: its kernels issue VALU instructions in three of four cycles
 // and the longer live ranges only cost them a wavefront or spills (18 tracers
-// on eight subdomains: 2.55 ms, against 3.2 ms with the lookahead).
+// on eight subdomains: 2.55 ms, against 3.2 ms with the lookahead).  All of
+// the row's loads are issued before anything else of it: left to the compiler,
+// the largest variants fetch a tracer at a time and wait for each (9 tracers
+// with budgets and diffusion, 700 x 600 x 30: 1492 us, 1185 with the barrier).
 template <typename TF>
 constexpr bool kRowAhead = sizeof(TF) == 8;
 
@@ -732,7 +733,10 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
     constexpr bool VF = decltype(vfc)::value, VR = decltype(vrc)::value;
     constexpr int w0 = R & 3, w1 = (R + 1) & 3, w2 = (R + 2) & 3, w3 = (R + 3) & 3;
     const int y = y0 - 2 + s;
-    if constexpr (!kRowAhead<TF>) load_row(y, buf);
+    if constexpr (!kRowAhead<TF>) {
+      load_row(y, buf);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     const int fl = (y >= 0 && y < NY) ? (buf.fl & cb.xin) : 0;  // raw masks of the cell
     const int fo = (fl | MB_XOUT) & cb.xm;                      // ... with the column bounds
 
@@ -860,10 +864,26 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
       if (dv.stop()) return;
     }
   }
-  step(Slot<0>{}, off, off, r, 0);
-  if (dv.stop()) return;
-  step(Slot<1>{}, off, off, r, 1);
-  step(Slot<2>{}, off, off, r, 2);
+  if constexpr (EXACT) {
+    step(Slot<0>{}, off, off, r, 0);
+    if (dv.stop()) return;
+    step(Slot<1>{}, off, off, r, 1);
+    step(Slot<2>{}, off, off, r, 2);
+  } else {
+    // one body for the three rows, the windows moved instead of renamed: less
+    // code (9 tracers: 55 -> 50 KB; 700 x 600 x 30: 1250 -> 1167 us)
+#pragma unroll 1
+    for (int s = 0; s < 3; s++) {
+      flw[3] = flw[0]; flw[0] = flw[1];
+      d1w[3] = d1w[0]; d1w[0] = d1w[1];
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        f1w[g][3] = f1w[g][0];
+        f1w[g][0] = f1w[g][1];
+      }
+      step(Slot<2>{}, off, off, r, s);
+    }
+  }
   step(Slot<3>{}, on, off, r, 3);
   if (dv.stop()) return;
   for (int s = 4; s < nsteps; s += 4) {
@@ -1061,7 +1081,10 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
     constexpr bool VF = decltype(vfc)::value, VR = decltype(vrc)::value;
     constexpr int w0 = R & 3, w1 = (R + 1) & 3, w2 = (R + 2) & 3, w3 = (R + 3) & 3;
     const int y = y0 - 2 + s;
-    if constexpr (!kRowAhead<TF>) load_row(y, buf);
+    if constexpr (!kRowAhead<TF>) {
+      load_row(y, buf);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     const int fl = (y >= 0 && y < NY) ? (buf.fl & cb.xin) : 0;  // raw masks of the cell
     const int fo = (fl | MB_XOUT) & cb.xm;                      // ... with the column bounds
 
@@ -1265,10 +1288,26 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
       if (dv.stop()) return;
     }
   }
-  step(Slot<0>{}, off, off, r, 0);
-  if (dv.stop()) return;
-  step(Slot<1>{}, off, off, r, 1);
-  step(Slot<2>{}, off, off, r, 2);
+  if constexpr (EXACT) {
+    step(Slot<0>{}, off, off, r, 0);
+    if (dv.stop()) return;
+    step(Slot<1>{}, off, off, r, 1);
+    step(Slot<2>{}, off, off, r, 2);
+  } else {
+    // (as in the first kernel)
+#pragma unroll 1
+    for (int s = 0; s < 3; s++) {
+      flw[3] = flw[0]; flw[0] = flw[1];
+      fow[3] = fow[0]; fow[0] = fow[1];
+      d3w[3] = d3w[0]; d3w[0] = d3w[1];
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        f3w[g][3] = f3w[g][0];
+        f3w[g][0] = f3w[g][1];
+      }
+      step(Slot<2>{}, off, off, r, s);
+    }
+  }
   step(Slot<3>{}, on, off, r, 3);
   if (dv.stop()) return;
   for (int s = 4; s < nsteps; s += 4) {

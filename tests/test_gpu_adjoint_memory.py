@@ -2,6 +2,8 @@
 checkpoint spacing bounds it, the default (which may take the whole window as
 one segment) holds no more than that takes, and a change of the mode gives it
 back.  Neither the spacing nor the mode changes a bit of the results."""
+import gc
+
 import pytest
 import torch
 
@@ -49,6 +51,8 @@ def test_memory_is_bounded_and_given_back(device):
         return free - torch.cuda.mem_get_info()[0], res
 
     adjoint64(ctx, 1, 1, F["dt"], f, lam, vel, gt.MUSCL, gt.MUSCL)  # (work fields of a step)
+    ctx.set_adjoint_mode(0)  # (nothing held)
+    gc.collect()
     torch.cuda.synchronize()
     start = torch.cuda.mem_get_info()[0]
     fields = {0: 5 + 2 + n // ck + ck - 1 + 4, 1: 5 + 2 + n // ck + ck - 1 + 4 * ck,

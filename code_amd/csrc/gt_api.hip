@@ -1093,7 +1093,7 @@ extern "C" int gt_uv_advect_3d(gt_ctx* c, double dt, const double* uu, const dou
       A.ndom = 1;
       A.ntracers = 1;
       if (c->tile >= 0) gt::strip_rows(c->tile, A.rows);
-      else gt::strip_auto_rows(A, 1);
+      else gt::strip_auto_rows(A, 1, 2.0);
       A.dt = dt;
       A.AH = 0.0;
       A.hscheme = hscheme; A.vscheme = vscheme;
@@ -1553,12 +1553,12 @@ static int batch_impl(int ndom, const gt_batch_domain* doms, int ntracers, doubl
     }
     A.ndom = nd;
     A.ntracers = ntracers;
-    // FP64: two tracers per wavefront (T and S) when there are two or more,
-    // unless the tuning asks for one
-    // (2 is no FP32 group: 3 stands for it)
-    const int group = sizeof(TF) == 4 && c0->group ? (c0->group == 2 ? 3 : c0->group)
-                      : c0->group == 1             ? 1
-                                                   : gt::strip_auto_group(A);
+    // (2 is no FP32 group: 3 stands for it; FP64 has 1 and 2)
+    const int group = c0->group == 0     ? gt::strip_auto_group(A)
+                      : c0->group == 1   ? 1
+                      : sizeof(TF) == 8  ? (ntracers >= 2 ? 2 : 1)
+                      : c0->group == 2   ? 3
+                                         : c0->group;
     if (c0->tile >= 0) gt::strip_rows(c0->tile, A.rows);
     else gt::strip_auto_rows(A, group);
     A.dt = dt; A.AH = AH;

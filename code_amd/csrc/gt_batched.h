@@ -72,11 +72,12 @@ struct FusedArgs {
 void strip_rows(int tile, int rows[2]);
 // the choice where the caller made none (gt_set_tuning): tracers per
 // wavefront, and rows per strip (4, 8, 16 or 32) given them; the caller has
-// filled doms, ndom and ntracers
+// filled doms, ndom and ntracers.  work: a wavefront's work against that of a
+// plain step
 template <typename TF>
 int strip_auto_group(const FusedArgs<TF>& a);
 template <typename TF>
-void strip_auto_rows(FusedArgs<TF>& a, int group);
+void strip_auto_rows(FusedArgs<TF>& a, int group, double work = 1.0);
 // the strip kernels are instantiated for hscheme == vscheme in UPSTREAM..P2_PDM
 bool fused_supported(int hscheme, int vscheme);
 // group: tracers per wavefront.  FP64: 1 or 2 (adv needs 1); FP32: 1, 3, 6 or 9.

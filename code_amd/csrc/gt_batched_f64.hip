@@ -36,48 +36,91 @@ static long strip_levels(const FusedArgs<TF>& a, int R, int n) {
   return items;
 }
 
-// The tracers per wavefront that cost least: a group's time is that of its
-// shared work and its slots, filled or not (1, 3, 6, 9 FP32 tracers: 27, 50,
-// 87, 128 in units of 10 us on the eight subdomains; 9 needs a grid that
-// fills the chip many times over, at 256 x 192 x 30 it takes 328 us for 18
-// tracers against 300 with 6).  Where even 4-row strips leave the chip short
-// of wavefronts a smaller group makes more of them (64 x 64 x 30 x 18: 60 us
-// with 6, 78 with 9; 6 tracers: 32 us with 3, 40 with 6).
+// The time of a launch of groups of g tracers and strips of R rows, in us: the
+// march is R + 4 steps, and a step takes what one wavefront needs for it alone
+// plus its share of all W wavefronts' work (times work, for the momentum
+// variants: 130 x 120 x 40 81 us with 8 rows, 92 with 4).  Fitted to P2-PDM from 20 x 16 x 5
+// to 700 x 600 x 30, 1 to 18 tracers, every g and R of 4, 8 and 16, to 10-15%;
+// the choices made from it are 2% slower than the best pair measured in the
+// mean, 15% at worst.
+template <typename TF>
+static double plan_cost(const FusedArgs<TF>& a, int g, int R, double work) {
+  struct Fit {
+    int g;
+    double alone, share;  // us, us per 1000 wavefronts
+  };
+  static const Fit f32[] = {{1, 2.0, 0.50}, {3, 2.85, 0.77}, {6, 3.9, 1.13}, {9, 4.6, 1.62}};
+  static const Fit f64[] = {{1, 2.1, 0.66}, {2, 2.7, 0.92}};
+  const Fit* f = sizeof(TF) == 4 ? f32 : f64;
+  while (f->g < g) f++;
+  const long W = strip_levels(a, R, (a.ntracers + g - 1) / g);
+  return (R + 4) * (f->alone + work * f->share * 1e-3 * (double)W);
+}
+template <typename TF>
+static int plan_rows(const FusedArgs<TF>& a, int g, double work, double* cost) {
+  int best = 16;
+  *cost = plan_cost(a, g, 16, work);
+  for (int R = 8; R >= 4; R /= 2) {
+    const double c = plan_cost(a, g, R, work);
+    if (c < *cost) {
+      *cost = c;
+      best = R;
+    }
+  }
+  return best;
+}
+
+// Tracers per wavefront: the group whose best strips cost least (FP32: 18 on
+// 100 x 100 x 20 62 us in groups of 3, 80 in groups of 9; 9 on 130 x 120 x 40
+// 82 with 9 and 4 rows, 106 with 9 and 8; 18 on 700 x 600 x 30 2.03 ms with 9,
+// 2.08 with 6).  FP64 takes two unless one is a tenth better (two tracers on
+// 20 x 16 x 5: 20 us one at a time, 26 together; on 400 x 400 x 40 two
+// together, 376).
 template <typename TF>
 int strip_auto_group(const FusedArgs<TF>& a) {
-  if constexpr (sizeof(TF) == 8) return a.ntracers >= 2 ? 2 : 1;
   if (a.ntracers == 1) return 1;
-  auto groups = [&](int g) { return (a.ntracers + g - 1) / g; };
-  const int c3 = groups(3) * 50, c6 = groups(6) * 87;
-  const int c9 = groups(9) * (strip_levels(a, 8, groups(9)) >= 32768 ? 128 : 138);
-  int g = c9 <= c6 && c9 <= c3 ? 9 : (c6 <= c3 ? 6 : 3);
-  while (g > 3 && strip_levels(a, 4, groups(g)) < 2560) g -= 3;
+  double cost, best = 0.0;
+  int g = 0;
+  auto take = [&](int group, double bias) {
+    (void)plan_rows(a, group, 1.0, &cost);
+    if (g == 0 || cost * bias < best) {
+      best = cost * bias;
+      g = group;
+    }
+  };
+  if constexpr (sizeof(TF) == 8) {
+    take(2, 1.0);
+    take(1, 1.1);
+  } else {
+    for (int group : {9, 6, 3, 1}) take(group, 1.0);
+  }
   return g;
 }
 
 // Strip heights.  A strip's march is a chain of rows + 4 steps, so where
 // 4-row strips fit the chip at once they are the fastest (100 x 100 x 20, one
-// FP64 tracer: 31 us, 38 with 8 rows, 61 with 16); beyond one round of
-// wavefronts the four ghost rows cost more than the shorter chain gives, and
-// taller strips follow (256 x 256 x 30: 16/8 92 us, 8/8 97, 16/16 99, 32/32
-// 141; 400 x 400 x 40 x 2: 16/16 371, 8/8 373, 32/32 389).  FP32 strips stay
-// at 8 rows longer (256 x 192 x 30 x 6: 8/8 105 us, 16/16 137; 512 x 384 x 30
-// x 6: 16/8 434, 16/16 455), and the largest grids take 32 (2000 x 1500 x 50
-// x 6: 9.9 ms against 10.3 with 16).
+// FP64 tracer: 31 us, 38 with 8 rows, 61 with 16); beyond a few wavefronts per
+// SIMD the four ghost rows cost more than the shorter chain gives, and taller
+// strips follow (256 x 256 x 30: 16/8 92 us, 8/8 97, 16/16 99, 32/32 141; 400
+// x 400 x 40 x 2: 16/16 371, 8/8 373, 32/32 389).  FP32 strips stay at 8 rows
+// longer (300 x 300 x 40 x 9: 8/8 366 us, 16/8 394; 700 x 600 x 30 x 6: 8/8
+// 854, 16/16 865), and the largest grids take 32 (2000 x 1500 x 50 x 6: 9.9 ms
+// against 10.0 with 16).
 template <typename TF>
-void strip_auto_rows(FusedArgs<TF>& a, int group) {
+void strip_auto_rows(FusedArgs<TF>& a, int group, double work) {
   const int ng = (a.ntracers + group - 1) / group;
-  const long i4 = strip_levels(a, 4, ng), i8 = strip_levels(a, 8, ng);
-  const long s8 = strip_levels(a, 8, 1);
-  const long upto8[2] = {sizeof(TF) == 8 ? 4096 : 8192, sizeof(TF) == 8 ? 8192 : 16384};
+  const long i8 = strip_levels(a, 8, ng), s8 = strip_levels(a, 8, 1);
+  double cost;
+  const bool shortest = plan_rows(a, group, work, &cost) == 4;
+  const long upto8[2] = {sizeof(TF) == 8 ? 4096 : 16384, sizeof(TF) == 8 ? 8192 : 16384};
   const bool tall[2] = {sizeof(TF) == 4 && i8 >= 65536, sizeof(TF) == 4 && s8 >= 200000};
   for (int p = 0; p < 2; p++)
-    a.rows[p] = i4 <= 3072 ? 4 : (i8 <= upto8[p] ? 8 : (tall[p] ? 32 : 16));
+    a.rows[p] = shortest ? 4 : (i8 <= upto8[p] ? 8 : (tall[p] ? 32 : 16));
 }
 template int strip_auto_group<double>(const FusedArgs<double>&);
 template int strip_auto_group<float>(const FusedArgs<float>&);
-template void strip_auto_rows<double>(FusedArgs<double>&, int);
-template void strip_auto_rows<float>(FusedArgs<float>&, int);
+template void strip_auto_rows<double>(FusedArgs<double>&, int, double);
+template void strip_auto_rows<float>(FusedArgs<float>&, int, double);
 
 hipError_t launch_fused_f64_g1(hipStream_t st, const FusedArgs<double>& a);
 hipError_t launch_fused_f64_g2(hipStream_t st, const FusedArgs<double>& a);

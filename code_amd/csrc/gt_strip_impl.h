@@ -553,6 +553,7 @@ __device__ __forceinline__ void sto(T* base, uint32_t off, T v) {
 // the row's loads are issued before anything else of it: left to the compiler,
 // the largest variants fetch a tracer at a time and wait for each (9 tracers
 // with budgets and diffusion, 700 x 600 x 30: 1492 us, 1185 with the barrier).
+// One tracer is better left alone (100 x 100 x 20: 20.4 us, 22.3 with it).
 template <typename TF>
 constexpr bool kRowAhead = sizeof(TF) == 8;
 
@@ -735,7 +736,7 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
     const int y = y0 - 2 + s;
     if constexpr (!kRowAhead<TF>) {
       load_row(y, buf);
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (G > 1) __builtin_amdgcn_sched_barrier(0);
     }
     const int fl = (y >= 0 && y < NY) ? (buf.fl & cb.xin) : 0;  // raw masks of the cell
     const int fo = (fl | MB_XOUT) & cb.xm;                      // ... with the column bounds
@@ -864,7 +865,7 @@ __device__ __forceinline__ void strip_uv(const FusedArgs<TF>& A, Div& dv) {
       if (dv.stop()) return;
     }
   }
-  if constexpr (EXACT) {
+  if constexpr (EXACT || G == 1) {
     step(Slot<0>{}, off, off, r, 0);
     if (dv.stop()) return;
     step(Slot<1>{}, off, off, r, 1);
@@ -1083,7 +1084,7 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
     const int y = y0 - 2 + s;
     if constexpr (!kRowAhead<TF>) {
       load_row(y, buf);
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (G > 1) __builtin_amdgcn_sched_barrier(0);
     }
     const int fl = (y >= 0 && y < NY) ? (buf.fl & cb.xin) : 0;  // raw masks of the cell
     const int fo = (fl | MB_XOUT) & cb.xm;                      // ... with the column bounds
@@ -1288,7 +1289,7 @@ __device__ __forceinline__ void strip_wvu(const FusedArgs<TF>& A, Div& dv) {
       if (dv.stop()) return;
     }
   }
-  if constexpr (EXACT) {
+  if constexpr (EXACT || G == 1) {
     step(Slot<0>{}, off, off, r, 0);
     if (dv.stop()) return;
     step(Slot<1>{}, off, off, r, 1);
